@@ -91,7 +91,7 @@ struct DevGemm {
     DevArray<GemmTile> tiles;
     DevArray<int> split;
     DevArray<RowMap> rowmap;
-    int ntiles = 0, nsplit = 0;
+    int ntiles = 0, nsplit = 0, rblocks = 0;
     void upload(const GemmList &g, hipStream_t s) {
         for (auto &x : g.groups) {
             if ((x.tm != 64 && x.tm != 128) || x.tn < 16 || x.tn > 128 || x.tn % 16 != 0)
@@ -110,6 +110,7 @@ struct DevGemm {
         split.upload(sp, s);
         ntiles = (int)g.tiles.size();
         nsplit = (int)sp.size();
+        rblocks = g.reduce_blocks();
     }
 };
 
@@ -451,20 +452,20 @@ static void sigma_stages(mq_plan *p, const double *x, double *y, int prec, hipEv
         if (prec == MQ_PREC_FP64) {
             check(launch_copy2d(p->reshape.p, (int)h.reshape.size(), x, p->prp.p, s, true), "copy psi");
             mark(2);
-            check(launch_gemm(p->g1.groups.p, p->g1.tiles.p, p->g1.ntiles, p->g1.split.p, p->g1.nsplit, p->prp.p,
+            check(launch_gemm(p->g1.groups.p, p->g1.tiles.p, p->g1.ntiles, p->g1.split.p, p->g1.nsplit, p->g1.rblocks, p->prp.p,
                               p->rb.p, p->t.p, p->ws.p, p->g1.rowmap.p, ST_SIGMA, s),
                   "gemm t");
             mark(3);
             check(launch_wapply(p->strips.p, p->packs.p, npacks(h.wapply), p->srcs.p, p->t.p, p->c.p, ST_SIGMA, s),
                   "W apply");
             mark(4);
-            check(launch_gemm(p->g2.groups.p, p->g2.tiles.p, p->g2.ntiles, p->g2.split.p, p->g2.nsplit, p->la.p,
+            check(launch_gemm(p->g2.groups.p, p->g2.tiles.p, p->g2.ntiles, p->g2.split.p, p->g2.nsplit, p->g2.rblocks, p->la.p,
                               p->c.p, p->tmp.p, p->ws.p, p->g2.rowmap.p, ST_SIGMA_OUT, s),
                   "gemm L");
         } else {
             check(launch_copy2d(p->reshape.p, (int)h.reshape.size(), x, p->prp32.p, s, true), "copy psi");
             mark(2);
-            check(launch_gemm(p->g1.groups.p, p->g1.tiles.p, p->g1.ntiles, p->g1.split.p, p->g1.nsplit, p->prp32.p,
+            check(launch_gemm(p->g1.groups.p, p->g1.tiles.p, p->g1.ntiles, p->g1.split.p, p->g1.nsplit, p->g1.rblocks, p->prp32.p,
                               p->rb32.p, p->t32.p, p->ws32.p, p->g1.rowmap.p, ST_SIGMA, s, x3),
                   "gemm t");
             mark(3);
@@ -472,7 +473,7 @@ static void sigma_stages(mq_plan *p, const double *x, double *y, int prec, hipEv
                                 s),
                   "W apply");
             mark(4);
-            check(launch_gemm(p->g2.groups.p, p->g2.tiles.p, p->g2.ntiles, p->g2.split.p, p->g2.nsplit, p->la32.p,
+            check(launch_gemm(p->g2.groups.p, p->g2.tiles.p, p->g2.ntiles, p->g2.split.p, p->g2.nsplit, p->g2.rblocks, p->la32.p,
                               p->c32.p, p->tmp.p, p->ws32.p, p->g2.rowmap.p, ST_SIGMA_OUT, s, x3),
                   "gemm L");
         }
@@ -483,27 +484,27 @@ static void sigma_stages(mq_plan *p, const double *x, double *y, int prec, hipEv
     if (prec == MQ_PREC_FP64) {
         check(launch_copy2d(p->reshape.p, (int)h.reshape.size(), x, p->prp.p, s, true), "reshape");
         mark(2);
-        check(launch_gemm(p->g1.groups.p, p->g1.tiles.p, p->g1.ntiles, p->g1.split.p, p->g1.nsplit, p->la.p,
+        check(launch_gemm(p->g1.groups.p, p->g1.tiles.p, p->g1.ntiles, p->g1.split.p, p->g1.nsplit, p->g1.rblocks, p->la.p,
                           p->prp.p, p->t.p, p->ws.p, p->g1.rowmap.p, ST_SIGMA, s),
               "gemm T");
         mark(3);
         check(launch_wapply(p->strips.p, p->packs.p, npacks(h.wapply), p->srcs.p, p->t.p, p->c.p, ST_SIGMA, s),
               "W apply");
         mark(4);
-        check(launch_gemm(p->g2.groups.p, p->g2.tiles.p, p->g2.ntiles, p->g2.split.p, p->g2.nsplit, p->c.p,
+        check(launch_gemm(p->g2.groups.p, p->g2.tiles.p, p->g2.ntiles, p->g2.split.p, p->g2.nsplit, p->g2.rblocks, p->c.p,
                           p->rb.p, y, p->ws.p, p->g2.rowmap.p, ST_SIGMA_OUT, s),
               "gemm R");
     } else {
         check(launch_copy2d(p->reshape.p, (int)h.reshape.size(), x, p->prp32.p, s, true), "reshape");
         mark(2);
-        check(launch_gemm(p->g1.groups.p, p->g1.tiles.p, p->g1.ntiles, p->g1.split.p, p->g1.nsplit, p->la32.p,
+        check(launch_gemm(p->g1.groups.p, p->g1.tiles.p, p->g1.ntiles, p->g1.split.p, p->g1.nsplit, p->g1.rblocks, p->la32.p,
                           p->prp32.p, p->t32.p, p->ws32.p, p->g1.rowmap.p, ST_SIGMA, s, x3),
               "gemm T");
         mark(3);
         check(launch_wapply(p->strips.p, p->packs.p, npacks(h.wapply), p->srcs.p, p->t32.p, p->c32.p, ST_SIGMA, s),
               "W apply");
         mark(4);
-        check(launch_gemm(p->g2.groups.p, p->g2.tiles.p, p->g2.ntiles, p->g2.split.p, p->g2.nsplit, p->c32.p,
+        check(launch_gemm(p->g2.groups.p, p->g2.tiles.p, p->g2.ntiles, p->g2.split.p, p->g2.nsplit, p->g2.rblocks, p->c32.p,
                           p->rb32.p, y, p->ws32.p, p->g2.rowmap.p, ST_SIGMA_OUT, s, x3),
               "gemm R");
     }
@@ -615,24 +616,24 @@ static void sigma_batch_launch(mq_plan *p, const double *L, const double *R, con
         const bool x3 = prec == MQ_PREC_BF16X3;
         if (prec == MQ_PREC_FP64) {
             check(launch_copy2d(B.reshape.p, (int)B.ncopies, X, B.prp.p, s, true), "copy psi");
-            check(launch_gemm(B.g1.groups.p, B.g1.tiles.p, B.g1.ntiles, B.g1.split.p, B.g1.nsplit, B.prp.p, p->rb.p,
+            check(launch_gemm(B.g1.groups.p, B.g1.tiles.p, B.g1.ntiles, B.g1.split.p, B.g1.nsplit, B.g1.rblocks, B.prp.p, p->rb.p,
                               B.t.p, B.ws.p, B.g1.rowmap.p, ST_SIGMA, s),
                   "gemm t");
             check(launch_wapply(p->strips.p, p->packs.p, npacks(h.wapply), p->srcs.p, B.t.p, B.c.p, ST_SIGMA, s, nvec,
                                 h.n_t, h.n_c),
                   "W apply");
-            check(launch_gemm(B.g2.groups.p, B.g2.tiles.p, B.g2.ntiles, B.g2.split.p, B.g2.nsplit, p->la.p, B.c.p,
+            check(launch_gemm(B.g2.groups.p, B.g2.tiles.p, B.g2.ntiles, B.g2.split.p, B.g2.nsplit, B.g2.rblocks, p->la.p, B.c.p,
                               A.tmp.p, B.ws.p, B.g2.rowmap.p, ST_SIGMA_OUT, s),
                   "gemm L");
         } else {
             check(launch_copy2d(B.reshape.p, (int)B.ncopies, X, B.prp32.p, s, true), "copy psi");
-            check(launch_gemm(B.g1.groups.p, B.g1.tiles.p, B.g1.ntiles, B.g1.split.p, B.g1.nsplit, B.prp32.p,
+            check(launch_gemm(B.g1.groups.p, B.g1.tiles.p, B.g1.ntiles, B.g1.split.p, B.g1.nsplit, B.g1.rblocks, B.prp32.p,
                               p->rb32.p, B.t32.p, B.ws32.p, B.g1.rowmap.p, ST_SIGMA, s, x3),
                   "gemm t");
             check(launch_wapply(p->strips.p, p->packs.p, npacks(h.wapply), p->srcs.p, B.t32.p, B.c32.p, ST_SIGMA, s,
                                 nvec, h.n_t, h.n_c),
                   "W apply");
-            check(launch_gemm(B.g2.groups.p, B.g2.tiles.p, B.g2.ntiles, B.g2.split.p, B.g2.nsplit, p->la32.p,
+            check(launch_gemm(B.g2.groups.p, B.g2.tiles.p, B.g2.ntiles, B.g2.split.p, B.g2.nsplit, B.g2.rblocks, p->la32.p,
                               B.c32.p, A.tmp.p, B.ws32.p, B.g2.rowmap.p, ST_SIGMA_OUT, s, x3),
                   "gemm L");
         }
@@ -641,24 +642,24 @@ static void sigma_batch_launch(mq_plan *p, const double *L, const double *R, con
     }
     if (prec == MQ_PREC_FP64) {
         check(launch_copy2d(B.reshape.p, (int)B.ncopies, X, B.prp.p, s, true), "reshape");
-        check(launch_gemm(B.g1.groups.p, B.g1.tiles.p, B.g1.ntiles, B.g1.split.p, B.g1.nsplit, p->la.p, B.prp.p,
+        check(launch_gemm(B.g1.groups.p, B.g1.tiles.p, B.g1.ntiles, B.g1.split.p, B.g1.nsplit, B.g1.rblocks, p->la.p, B.prp.p,
                           B.t.p, B.ws.p, B.g1.rowmap.p, ST_SIGMA, s),
               "gemm T");
         check(launch_wapply(p->strips.p, p->packs.p, npacks(h.wapply), p->srcs.p, B.t.p, B.c.p, ST_SIGMA, s, nvec,
                             h.n_t, h.n_c),
               "W apply");
-        check(launch_gemm(B.g2.groups.p, B.g2.tiles.p, B.g2.ntiles, B.g2.split.p, B.g2.nsplit, B.c.p, p->rb.p, Y,
+        check(launch_gemm(B.g2.groups.p, B.g2.tiles.p, B.g2.ntiles, B.g2.split.p, B.g2.nsplit, B.g2.rblocks, B.c.p, p->rb.p, Y,
                           B.ws.p, B.g2.rowmap.p, ST_SIGMA_OUT, s),
               "gemm R");
     } else {
         check(launch_copy2d(B.reshape.p, (int)B.ncopies, X, B.prp32.p, s, true), "reshape");
-        check(launch_gemm(B.g1.groups.p, B.g1.tiles.p, B.g1.ntiles, B.g1.split.p, B.g1.nsplit, p->la32.p,
+        check(launch_gemm(B.g1.groups.p, B.g1.tiles.p, B.g1.ntiles, B.g1.split.p, B.g1.nsplit, B.g1.rblocks, p->la32.p,
                           B.prp32.p, B.t32.p, B.ws32.p, B.g1.rowmap.p, ST_SIGMA, s, prec == MQ_PREC_BF16X3),
               "gemm T");
         check(launch_wapply(p->strips.p, p->packs.p, npacks(h.wapply), p->srcs.p, B.t32.p, B.c32.p, ST_SIGMA, s,
                             nvec, h.n_t, h.n_c),
               "W apply");
-        check(launch_gemm(B.g2.groups.p, B.g2.tiles.p, B.g2.ntiles, B.g2.split.p, B.g2.nsplit, B.c32.p,
+        check(launch_gemm(B.g2.groups.p, B.g2.tiles.p, B.g2.ntiles, B.g2.split.p, B.g2.nsplit, B.g2.rblocks, B.c32.p,
                           p->rb32.p, Y, B.ws32.p, B.g2.rowmap.p, ST_SIGMA_OUT, s, prec == MQ_PREC_BF16X3),
               "gemm R");
     }
@@ -846,7 +847,7 @@ int mq_gemm_f64(mq_ctx *ctx, int transA, int transB, int M, int N, int K, const 
         dg.upload(gl, ctx->stream);
         DevArray<double> ws;
         ws.alloc((size_t)gl.ws);
-        check(launch_gemm(dg.groups.p, dg.tiles.p, dg.ntiles, dg.split.p, dg.nsplit, A, B, C, ws.p, dg.rowmap.p, ST_MISC,
+        check(launch_gemm(dg.groups.p, dg.tiles.p, dg.ntiles, dg.split.p, dg.nsplit, dg.rblocks, A, B, C, ws.p, dg.rowmap.p, ST_MISC,
                           ctx->stream),
               "gemm");
         check(hipStreamSynchronize(ctx->stream), "gemm sync");
@@ -909,7 +910,7 @@ int mq_gemm_f64_noalloc(mq_ctx *ctx, int transA, int transB, int M, int N, int K
                   "tile upload");
         check(launch_gemm(reinterpret_cast<const GemmGroup *>(base + o_grp),
                           reinterpret_cast<const GemmTile *>(base + o_til), (int)gl.tiles.size(),
-                          reinterpret_cast<const int *>(base + o_sp), (int)sp.size(), A, B, C,
+                          reinterpret_cast<const int *>(base + o_sp), (int)sp.size(), gl.reduce_blocks(), A, B, C,
                           reinterpret_cast<double *>(base + o_ws), nullptr, ST_MISC, s),
               "gemm");
         // the host task lists must outlive their copies
@@ -945,7 +946,7 @@ int mq_gemm_f32(mq_ctx *ctx, int transA, int transB, int M, int N, int K, const 
         dg.upload(gl, ctx->stream);
         DevArray<float> ws;
         ws.alloc((size_t)gl.ws);
-        check(launch_gemm(dg.groups.p, dg.tiles.p, dg.ntiles, dg.split.p, dg.nsplit, A, B, C, ws.p, dg.rowmap.p, ST_MISC,
+        check(launch_gemm(dg.groups.p, dg.tiles.p, dg.ntiles, dg.split.p, dg.nsplit, dg.rblocks, A, B, C, ws.p, dg.rowmap.p, ST_MISC,
                           ctx->stream, bf16x3 != 0),
               "gemm");
         check(hipStreamSynchronize(ctx->stream), "gemm sync");
@@ -1051,24 +1052,24 @@ int mq_boundary_step(mq_plan *plan, const double *in, const double *A, double *o
         if (h.kind == PLAN_LSTEP) {
             arrange_left(plan, in, s);
             check(launch_gemm(plan->g1.groups.p, plan->g1.tiles.p, plan->g1.ntiles, plan->g1.split.p,
-                              plan->g1.nsplit, plan->la.p, plan->prp.p, plan->t.p, plan->ws.p, plan->g1.rowmap.p, ST_STEP, s),
+                              plan->g1.nsplit, plan->g1.rblocks, plan->la.p, plan->prp.p, plan->t.p, plan->ws.p, plan->g1.rowmap.p, ST_STEP, s),
                   "gemm T");
             check(launch_wapply(plan->strips.p, plan->packs.p, npacks(h.wapply), plan->srcs.p, plan->t.p, plan->c.p,
                                 ST_STEP, s),
                   "W apply");
             check(launch_gemm(plan->g2.groups.p, plan->g2.tiles.p, plan->g2.ntiles, plan->g2.split.p,
-                              plan->g2.nsplit, plan->c.p, A, plan->tmp.p, plan->ws.p, plan->g2.rowmap.p, ST_STEP_OUT, s),
+                              plan->g2.nsplit, plan->g2.rblocks, plan->c.p, A, plan->tmp.p, plan->ws.p, plan->g2.rowmap.p, ST_STEP_OUT, s),
                   "gemm out");
         } else {
             check(launch_copy2d(plan->arrR.p, (int)h.arrR.size(), in, plan->rb.p, s), "arrange R");
             check(launch_gemm(plan->g1.groups.p, plan->g1.tiles.p, plan->g1.ntiles, plan->g1.split.p,
-                              plan->g1.nsplit, A, plan->rb.p, plan->t.p, plan->ws.p, plan->g1.rowmap.p, ST_STEP, s),
+                              plan->g1.nsplit, plan->g1.rblocks, A, plan->rb.p, plan->t.p, plan->ws.p, plan->g1.rowmap.p, ST_STEP, s),
                   "gemm t");
             check(launch_wapply(plan->strips.p, plan->packs.p, npacks(h.wapply), plan->srcs.p, plan->t.p, plan->c.p,
                                 ST_STEP, s),
                   "W apply");
             check(launch_gemm(plan->g2.groups.p, plan->g2.tiles.p, plan->g2.ntiles, plan->g2.split.p,
-                              plan->g2.nsplit, plan->c.p, plan->prp.p, plan->tmp.p, plan->ws.p, plan->g2.rowmap.p, ST_STEP_OUT, s),
+                              plan->g2.nsplit, plan->g2.rblocks, plan->c.p, plan->prp.p, plan->tmp.p, plan->ws.p, plan->g2.rowmap.p, ST_STEP_OUT, s),
                   "gemm out");
         }
         check(launch_copy2d(plan->scatter.p, (int)h.scatter.size(), plan->tmp.p, out, s), "scatter");
@@ -1092,7 +1093,7 @@ int mq_diagonal(mq_plan *plan, const double *L, const double *R, double *diag) {
         check(launch_wapply(plan->strips.p, plan->packs.p, npacks(h.wapply), plan->srcs.p, plan->la.p, plan->t.p,
                             ST_MISC, s),
               "diagonal W apply");
-        check(launch_gemm(plan->g2.groups.p, plan->g2.tiles.p, plan->g2.ntiles, plan->g2.split.p, plan->g2.nsplit,
+        check(launch_gemm(plan->g2.groups.p, plan->g2.tiles.p, plan->g2.ntiles, plan->g2.split.p, plan->g2.nsplit, plan->g2.rblocks,
                           plan->t.p, plan->rb.p, diag, plan->ws.p, plan->g2.rowmap.p, ST_MISC, s),
               "diagonal gemm");
         return MQ_OK;

@@ -29,14 +29,16 @@ hipError_t launch_wapply(const Strip *strips, const int *packs, int npacks, cons
                          int stage, hipStream_t s, int nvec = 1, int64_t src_stride = 0, int64_t dst_stride = 0);
 // grouped GEMM over a plan's tile list (FP64; FP32 operands with FP32 or FP64 output,
 // multiplied in FP32 or, with bf16x3, as three bf16 products accumulated in FP32);
+// split_gids, nsplit: the groups with split-K partials; rblocks: workgroups of 256 that
+// cover the largest one's elements (GemmList::reduce_blocks);
 // rowmap: the row placements of groups with rowmap > 0 (may be null when none has)
-hipError_t launch_gemm(const GemmGroup *groups, const GemmTile *tiles, int ntiles, const int *split_gids, int nsplit,
+hipError_t launch_gemm(const GemmGroup *groups, const GemmTile *tiles, int ntiles, const int *split_gids, int nsplit, int rblocks,
                        const double *A, const double *B, double *C, double *W, const RowMap *rowmap, int stage,
                        hipStream_t s);
-hipError_t launch_gemm(const GemmGroup *groups, const GemmTile *tiles, int ntiles, const int *split_gids, int nsplit,
+hipError_t launch_gemm(const GemmGroup *groups, const GemmTile *tiles, int ntiles, const int *split_gids, int nsplit, int rblocks,
                        const float *A, const float *B, float *C, float *W, const RowMap *rowmap, int stage,
                        hipStream_t s, bool bf16x3 = false);
-hipError_t launch_gemm(const GemmGroup *groups, const GemmTile *tiles, int ntiles, const int *split_gids, int nsplit,
+hipError_t launch_gemm(const GemmGroup *groups, const GemmTile *tiles, int ntiles, const int *split_gids, int nsplit, int rblocks,
                        const float *A, const float *B, double *C, float *W, const RowMap *rowmap, int stage,
                        hipStream_t s, bool bf16x3 = false);
 hipError_t launch_multidot(const double *const *xs, const double *const *ys, int npairs, int64_t n, int nblocks,

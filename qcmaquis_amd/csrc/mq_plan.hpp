@@ -84,10 +84,6 @@ struct GemmTile {
     int g;
     int mt, nt, ks;
 };
-// partial-sum reduction of one split group: C = sum_s part[s]
-struct ReduceTask {
-    int g;
-};
 
 // dst(rows x cols, ldd) = sum over sources of coef * src(rows x cols, lds)
 struct Strip {
@@ -114,6 +110,13 @@ struct GemmList {
         double f = 0;
         for (auto &g : groups) f += 2.0 * g.M * g.N * g.K;
         return f;
+    }
+    // workgroups of 256 elements that cover the largest split group's output
+    int reduce_blocks() const {
+        int64_t b = 0;
+        for (auto &g : groups)
+            if (g.split > 1) b = std::max(b, ((int64_t)g.M * g.N + 255) / 256);
+        return (int)b;
     }
 };
 // Consecutive strips are run in packs of one workgroup each: a pack is either
