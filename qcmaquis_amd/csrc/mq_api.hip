@@ -146,12 +146,11 @@ struct mq_plan {
     DevArray<float> la32, rb32, prp32, t32, c32, ws32;
     bool conv32 = false;  // la32 / rb32 hold the current binding
     // Davidson workspace
-    DevArray<double> jd_vecs, jd_partial, jd_coef;
-    DevArray<const double *> jd_ptrs;
+    DevArray<double> jd_vecs, jd_partial;
     int jd_cap = 0;
-    // pinned host staging of the Davidson coefficients / pointers / partial sums
-    double *h_coef = nullptr, *h_partial = nullptr;
-    const double **h_ptrs = nullptr;
+    // partial sums of dot products, written by the kernels (pinned host memory)
+    double *h_partial = nullptr;
+    hipEvent_t jd_event = nullptr;
     // several vectors per launch (mq_sigma_batch): replicated task lists per batch
     // size, and per-vector copies of the psi, T and C arenas for the largest size used
     struct BatchLists {  // the W application reuses the plan's own strips for every vector
@@ -177,9 +176,8 @@ struct mq_plan {
     double solve_info[4] = {0, 0, 0, 0};
     ~mq_plan() {
         if (gexec) (void)hipGraphExecDestroy(gexec);
-        if (h_coef) (void)hipHostFree(h_coef);
         if (h_partial) (void)hipHostFree(h_partial);
-        if (h_ptrs) (void)hipHostFree((void *)h_ptrs);
+        if (jd_event) (void)hipEventDestroy(jd_event);
     }
 };
 
@@ -1107,83 +1105,67 @@ int mq_diagonal(mq_plan *plan, const double *L, const double *R, double *diag) {
 // ------------------------------------------------------------------ Jacobi-Davidson
 namespace {
 
-// Davidson vector operations on the plan's stream.  Pointer lists and
-// coefficients are staged in pinned host slots that stay untouched until the
-// next synchronisation, so linear combinations are enqueued without waiting;
-// only dot products synchronise (one launch for a whole batch of pairs).
-constexpr int kJdSlots = 4096, kJdPartialPairs = 128, kJdBlocks = 256;
+// Davidson vector operations on the plan's stream.  Linear combinations are enqueued
+// without waiting; dot products synchronise (once for a batch of up to kJdPartialPairs
+// pairs), their per-block partials written by the kernels to pinned host memory.
+constexpr int kJdPartialPairs = 128, kJdBlocks = 256;
 
 struct JD {
     mq_plan *p;
     hipStream_t s;
     int64_t n;
     int nblk;
-    int ptr_used = 0, coef_used = 0;
 
     double *vec(int i) { return p->jd_vecs.p + (int64_t)i * n; }
 
     void init() {
-        if (!p->h_coef) {
-            check(hipHostMalloc((void **)&p->h_coef, sizeof(double) * kJdSlots), "pinned coef");
+        if (!p->h_partial) {
             check(hipHostMalloc((void **)&p->h_partial, sizeof(double) * kJdPartialPairs * kJdBlocks),
                   "pinned partials");
-            check(hipHostMalloc((void **)&p->h_ptrs, sizeof(double *) * kJdSlots), "pinned ptrs");
-            p->jd_partial.alloc((size_t)kJdPartialPairs * kJdBlocks);
-            p->jd_coef.alloc(kJdSlots);
-            p->jd_ptrs.alloc(kJdSlots);
         }
+        if (!p->jd_event) check(hipEventCreateWithFlags(&p->jd_event, hipEventDisableTiming), "davidson event");
     }
-    const double **stage_ptrs(const std::vector<const double *> &v, int *slot) {
-        if (ptr_used + (int)v.size() > kJdSlots) sync();
-        *slot = ptr_used;
-        for (size_t i = 0; i < v.size(); ++i) p->h_ptrs[ptr_used + i] = v[i];
-        check(hipMemcpyAsync(p->jd_ptrs.p + ptr_used, p->h_ptrs + ptr_used, sizeof(double *) * v.size(),
-                             hipMemcpyHostToDevice, s),
-              "stage ptrs");
-        ptr_used += (int)v.size();
-        return p->jd_ptrs.p + *slot;
+    void sync() { check(hipStreamSynchronize(s), "davidson sync"); }
+    // row k of the pinned partials, summed in a fixed order
+    double host_sum(int k) const {
+        long double acc = 0;
+        for (int b = 0; b < nblk; ++b) acc += p->h_partial[(size_t)k * nblk + b];
+        return (double)acc;
     }
-    void sync() {
-        check(hipStreamSynchronize(s), "davidson sync");
-        ptr_used = coef_used = 0;
-    }
-    // dots of pairs (x_k, y_k), summed on the host in a fixed order (one
-    // synchronisation per kJdPartialPairs pairs)
+    // dots of pairs (x_k, y_k)
     std::vector<double> dots(const std::vector<const double *> &xs, const std::vector<const double *> &ys) {
         const int np_all = (int)xs.size();
         std::vector<double> r(np_all, 0.0);
         for (int k0 = 0; k0 < np_all; k0 += kJdPartialPairs) {
             const int np = std::min(kJdPartialPairs, np_all - k0);
-            std::vector<const double *> ptrs(xs.begin() + k0, xs.begin() + k0 + np);
-            ptrs.insert(ptrs.end(), ys.begin() + k0, ys.begin() + k0 + np);
-            int slot;
-            const double *const *d = stage_ptrs(ptrs, &slot);
-            check(launch_multidot(d, d + np, np, n, nblk, p->jd_partial.p, s), "multidot");
-            check(hipMemcpyAsync(p->h_partial, p->jd_partial.p, sizeof(double) * np * nblk, hipMemcpyDeviceToHost,
-                                 s),
-                  "dot partials");
-            sync();
-            for (int k = 0; k < np; ++k) {
-                long double acc = 0;
-                for (int b = 0; b < nblk; ++b) acc += p->h_partial[(size_t)k * nblk + b];
-                r[k0 + k] = (double)acc;
+            for (int q0 = 0; q0 < np; q0 += kCombMax) {
+                const int nq = std::min(kCombMax, np - q0);
+                PairArgs a{};
+                for (int q = 0; q < nq; ++q) {
+                    a.x[q] = xs[k0 + q0 + q];
+                    a.y[q] = ys[k0 + q0 + q];
+                }
+                check(launch_multidot(a, nq, n, nblk, p->h_partial + (size_t)q0 * nblk, s), "multidot");
             }
+            sync();
+            for (int k = 0; k < np; ++k) r[k0 + k] = host_sum(k);
         }
         return r;
     }
     double dot(const double *x, const double *y) { return dots({x}, {y})[0]; }
-    // out = beta*out + sum c_j v_j, enqueued without waiting
+    // out = beta*out + sum c_j v_j, enqueued without waiting (out is none of the v_j
+    // beyond the first kCombMax)
     void lincomb(const std::vector<const double *> &vs, const std::vector<double> &c, double beta, double *out) {
-        int nv = (int)vs.size();
-        if (coef_used + nv > kJdSlots || ptr_used + nv > kJdSlots) sync();
-        int slot;
-        const double *const *d = stage_ptrs(vs, &slot);
-        int cs = coef_used;
-        for (int j = 0; j < nv; ++j) p->h_coef[cs + j] = c[j];
-        check(hipMemcpyAsync(p->jd_coef.p + cs, p->h_coef + cs, sizeof(double) * nv, hipMemcpyHostToDevice, s),
-              "stage coef");
-        coef_used += nv;
-        check(launch_lincomb(d, p->jd_coef.p + cs, nv, n, beta, out, s), "lincomb");
+        const int nv = (int)vs.size();
+        for (int j0 = 0; j0 < nv; j0 += kCombMax) {
+            const int nj = std::min(kCombMax, nv - j0);
+            CombArgs a{};
+            for (int j = 0; j < nj; ++j) {
+                a.v[j] = vs[j0 + j];
+                a.c[j] = c[j0 + j];
+            }
+            check(launch_lincomb(a, nj, n, j0 ? 1.0 : beta, out, s), "lincomb");
+        }
     }
 };
 
@@ -1283,73 +1265,82 @@ extern "C" int mq_jacobi_davidson(mq_plan *plan, const double *L, const double *
         jd.nblk = (int)std::max<int64_t>(1, std::min<int64_t>(kJdBlocks, (jd.n + 255) / 256));
         jd.init();
         const int64_t n = jd.n;
-        int need = 2 * max_iter + 2;
+        const int need = 2 * max_iter + 2 + n_ortho;
         if (plan->jd_cap < need) {
             plan->jd_vecs.alloc((size_t)need * n);
             plan->jd_cap = need;
         }
         auto V = [&](int i) { return jd.vec(i); };
         auto VA = [&](int i) { return jd.vec(max_iter + i); };
-        double *u = jd.vec(2 * max_iter), *uA = jd.vec(2 * max_iter + 1);
-        std::vector<double> oo(n_ortho);
-        for (int k = 0; k < n_ortho; ++k) oo[k] = jd.dot(ortho[k], ortho[k]);
-        auto project = [&](double *t) {  // SingleSiteVS::project (ietl_lanczos_solver.h:90-95)
+        double *u = jd.vec(2 * max_iter), *uA = jd.vec(2 * max_iter + 1), *O = jd.vec(2 * max_iter + 2);
+        // partials of the orthonormalisation: the dots of t before it, after each update and
+        // around the projection (rows: t.t, then one per basis vector), and of the residual
+        const size_t rows = (size_t)std::max(max_iter, n_ortho) + 1;
+        const size_t part = (4 * rows + 3) * jd.nblk;
+        if (plan->jd_partial.n < part + n_ortho) plan->jd_partial.alloc(part + n_ortho);
+        double *p0 = plan->jd_partial.p, *p1 = p0 + rows * jd.nblk, *p2 = p1 + rows * jd.nblk,
+               *p3 = p2 + rows * jd.nblk, *pr = p3 + rows * jd.nblk, *ow = pr + 3 * jd.nblk;
+        if (n_ortho > 0) {
+            std::vector<const double *> o(ortho, ortho + n_ortho);
+            std::vector<double> oo = jd.dots(o, o);
+            for (auto &x : oo) x = 1.0 / x;
+            for (int k = 0; k < n_ortho; ++k)
+                check(hipMemcpyAsync(O + (int64_t)k * n, ortho[k], sizeof(double) * n, hipMemcpyDeviceToDevice, jd.s),
+                      "ortho");
+            check(hipMemcpyAsync(ow, oo.data(), sizeof(double) * n_ortho, hipMemcpyHostToDevice, jd.s), "ortho norms");
+            jd.sync();  // oo goes out of scope
+        }
+        // SingleSiteVS::project (ietl_lanczos_solver.h:90-95); leaves the dots of t in p3
+        auto project = [&](double *t) {
             if (n_ortho == 0) return;
-            std::vector<const double *> xs, ys;
-            for (int k = 0; k < n_ortho; ++k) {
-                xs.push_back(ortho[k]);
-                ys.push_back(t);
+            check(launch_orth(ORTH_DOTS, O, n, n_ortho, t, nullptr, nullptr, nullptr, nullptr, nullptr, true, jd.nblk,
+                              p2, jd.s),
+                  "project");
+            check(launch_orth(ORTH_UPDATE, O, n, n_ortho, t, nullptr, nullptr, ow, p2, nullptr, true, jd.nblk, p3,
+                              jd.s),
+                  "project");
+        };
+        // orthonormalise t = V(m), its dots in p0 (jacobi.h:384-393: Gram-Schmidt, repeated
+        // when the norm drops below a quarter of its value), on the device alone
+        auto orthonormalise = [&](int m) {
+            double *t = V(m);
+            if (m > 0) {
+                check(launch_orth(ORTH_UPDATE, V(0), n, m, t, nullptr, nullptr, nullptr, p0, nullptr, true, jd.nblk,
+                                  p1, jd.s),
+                      "orthogonalise");
+                check(launch_orth(ORTH_UPDATE, V(0), n, m, t, nullptr, nullptr, nullptr, p1, p0, true, jd.nblk, p2,
+                                  jd.s),
+                      "orthogonalise");
             }
-            std::vector<double> d = jd.dots(xs, ys), c(n_ortho);
-            for (int k = 0; k < n_ortho; ++k) c[k] = -d[k] / oo[k];
-            jd.lincomb(std::vector<const double *>(ortho, ortho + n_ortho), c, 1.0, t);
+            project(t);
+            if (n_ortho > 0)
+                check(launch_normalise(t, n, jd.nblk, nullptr, p3, nullptr, jd.s), "normalise");
+            else if (m > 0)
+                check(launch_normalise(t, n, jd.nblk, p0, p1, p2, jd.s), "normalise");
+            else
+                check(launch_normalise(t, n, jd.nblk, nullptr, p0, nullptr, jd.s), "normalise");
         };
         check(hipMemcpyAsync(V(0), x0, sizeof(double) * n, hipMemcpyDeviceToDevice, jd.s), "x0");
         project(V(0));
+        check(launch_orth(ORTH_DOTS, V(0), n, 0, V(0), nullptr, nullptr, nullptr, nullptr, nullptr, true, jd.nblk, p0,
+                          jd.s),
+              "norm");
+        orthonormalise(0);
         std::vector<double> M((size_t)max_iter * max_iter, 0.0);
         int it = 0;
         double theta = 0;
         while (true) {
-            // orthogonalise t against V (jacobi.h:384-393: Gram-Schmidt, repeated when the
-            // norm drops below a quarter of its value), then normalise
-            double *t = V(it);
-            std::vector<const double *> xs{t}, ys{t};
-            for (int i = 0; i < it; ++i) {
-                xs.push_back(V(i));
-                ys.push_back(t);
-            }
-            std::vector<double> d = jd.dots(xs, ys);
-            const double tau = std::sqrt(d[0]);
-            double nt2 = d[0];
-            for (int pass = 0; pass < 2 && it > 0; ++pass) {
-                std::vector<const double *> vv;
-                std::vector<double> c;
-                for (int i = 0; i < it; ++i) {
-                    vv.push_back(V(i));
-                    c.push_back(-d[1 + i]);
-                }
-                jd.lincomb(vv, c, 1.0, t);
-                d = jd.dots(xs, ys);
-                nt2 = d[0];
-                if (std::sqrt(nt2) >= 0.25 * tau) break;
-            }
-            if (n_ortho > 0) {
-                project(t);
-                nt2 = jd.dot(t, t);
-            }
-            const double nt = std::sqrt(nt2);
-            jd.lincomb({t}, {1.0 / nt - 1.0}, 1.0, t);
-            solver_sigma(plan, L, R, t, VA(it), prec);
+            solver_sigma(plan, L, R, V(it), VA(it), prec);
             // Rayleigh column (jacobi.h:401-402)
-            xs.clear();
-            ys.clear();
-            for (int i = 0; i <= it; ++i) {
-                xs.push_back(V(i));
-                ys.push_back(VA(it));
+            const int dim = it + 1;
+            for (int i0 = 0; i0 < dim; i0 += kJdPartialPairs) {
+                const int ni = std::min(kJdPartialPairs, dim - i0);
+                check(launch_orth(ORTH_DOTS, V(i0), n, ni, VA(it), nullptr, nullptr, nullptr, nullptr, nullptr, false,
+                                  jd.nblk, plan->h_partial, jd.s),
+                      "Rayleigh column");
+                jd.sync();
+                for (int i = 0; i < ni; ++i) M[(size_t)it * max_iter + i0 + i] = jd.host_sum(i);
             }
-            std::vector<double> col = jd.dots(xs, ys);
-            for (int i = 0; i <= it; ++i) M[(size_t)it * max_iter + i] = col[i];
-            int dim = it + 1;
             std::vector<double> A((size_t)dim * dim);
             for (int i = 0; i < dim; ++i)
                 for (int j = 0; j <= i; ++j) {
@@ -1369,23 +1360,38 @@ extern "C" int mq_jacobi_davidson(mq_plan *plan, const double *L, const double *
                 if (std::fabs(sv[i]) > std::fabs(sv[big])) big = i;
             if (sv[big] < 0)
                 for (auto &v : sv) v = -v;
-            std::vector<const double *> vv, va;
-            for (int j = 0; j < dim; ++j) {
-                vv.push_back(V(j));
-                va.push_back(VA(j));
+            // u = V sv, r = project(VA sv) - theta u, with |r|, r.u and u.u
+            for (int j0 = 0; j0 < dim; j0 += kCombMax) {
+                const int nj = std::min(kCombMax, dim - j0);
+                const bool last = j0 + nj == dim;
+                RitzArgs c{};
+                for (int j = 0; j < nj; ++j) c.c[j] = sv[j0 + j];
+                check(launch_ritz(c, nj, V(j0), VA(j0), n, last && n_ortho == 0 ? theta : 0.0, j0 == 0, last, u, uA,
+                                  jd.nblk, pr, plan->h_partial, jd.s),
+                      "Ritz vector");
             }
-            jd.lincomb(vv, sv, 0.0, u);
-            jd.lincomb(va, sv, 0.0, uA);
-            project(uA);
-            jd.lincomb({u}, {-theta}, 1.0, uA);  // r = uA - theta u
+            if (n_ortho > 0) {
+                project(uA);
+                jd.lincomb({u}, {-theta}, 1.0, uA);
+                check(launch_multidot(PairArgs{{uA, uA, u}, {uA, u, u}}, 3, n, jd.nblk, plan->h_partial, jd.s),
+                      "residual");
+                check(launch_multidot(PairArgs{{uA, uA, u}, {uA, u, u}}, 3, n, jd.nblk, pr, jd.s), "residual");
+            }
+            check(hipEventRecord(plan->jd_event, jd.s), "record");
             ++it;
-            // |r|, r.u and u.u in one batch: convergence test and correction t = -r + (r.u)/(u.u) u
-            std::vector<double> rr = jd.dots({uA, uA, u}, {uA, u, u});
-            double rn = std::sqrt(rr[0]);
+            if (it < max_iter) {
+                // the next basis vector, t = -r + (r.u)/(u.u) u orthonormalised, is formed while the
+                // host tests the residual (only u and r are used when the solve ends here)
+                check(launch_orth(ORTH_CORRECTION, V(0), n, it, V(it), u, uA, nullptr, pr, nullptr, true, jd.nblk, p0,
+                                  jd.s),
+                      "correction");
+                orthonormalise(it);
+            }
+            check(hipEventSynchronize(plan->jd_event), "residual");
+            const double rn = std::sqrt(jd.host_sum(0));
             if (rn <= ptol * std::fabs(theta) || rn < ptol || it >= max_iter ||
                 stall.update(rn / std::max(std::fabs(theta), 1e-300)))
                 break;
-            jd.lincomb({uA, u}, {-1.0, rr[1] / rr[2]}, 0.0, V(it));
         }
         const double theta_form = theta;
         const int its_form = it;

@@ -621,12 +621,14 @@ __global__ void __launch_bounds__(256) k_split_reduce(const GemmGroup *__restric
 }
 
 // ------------------------------------------------------------------ vector kernels (Davidson)
-// Partial dot products of K vector pairs; block b writes its partial for pair p.
-__global__ void __launch_bounds__(256) k_multidot(const double *const *__restrict__ xs,
-                                                  const double *const *__restrict__ ys, int64_t n,
-                                                  double *__restrict__ partial) {
+// Pointers and coefficients travel as kernel arguments, and partial sums may go
+// straight to pinned host memory: the small copies they replace cost 2.3 us of GPU time
+// and a submission each, twenty per Jacobi-Davidson iteration.
+
+// Partial dot products of vector pairs; block b writes its partial for pair p.
+__global__ void __launch_bounds__(256) k_multidot(const PairArgs a, int64_t n, double *__restrict__ partial) {
     const int p = blockIdx.y;
-    const double *x = xs[p], *y = ys[p];
+    const double *x = a.x[p], *y = a.y[p];
     __shared__ double red[256];
     double acc = 0.0;
     for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < n; e += (int64_t)gridDim.x * blockDim.x)
@@ -641,14 +643,148 @@ __global__ void __launch_bounds__(256) k_multidot(const double *const *__restric
 }
 
 // out = sum_j c_j * v_j  (+ beta * out if beta != 0)
-__global__ void __launch_bounds__(256) k_lincomb(const double *const *__restrict__ vs,
-                                                 const double *__restrict__ coef, int nv, int64_t n, double beta,
+__global__ void __launch_bounds__(256) k_lincomb(const CombArgs a, int nv, int64_t n, double beta,
                                                  double *__restrict__ out) {
     for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < n; e += (int64_t)gridDim.x * blockDim.x) {
         double acc = (beta != 0.0) ? beta * out[e] : 0.0;
-        for (int j = 0; j < nv; ++j) acc = fma(coef[j], vs[j][e], acc);
+        for (int j = 0; j < nv; ++j) acc = fma(a.c[j], a.v[j][e], acc);
         out[e] = acc;
     }
+}
+
+// ---- one orthonormalisation step without the host (Jacobi-Davidson)
+// Gram-Schmidt of t against m basis vectors needs its dot products, the update, the new
+// dot products, perhaps a second update, and the norm.  Each is a kernel whose blocks
+// sum the previous one's per-block partials themselves, so the host waits for none of
+// them.  What bounds them is latency: at L=24 m=512 a vector is 2.7 MB and a kernel a
+// few us; the host round trips they replace were about 20 us each.  Ten iterations at
+// L=8 m=64 (2,000 elements): 1,948 us with host-driven steps, 1,118 us so; at L=24
+// m=512 54.0 -> 52.9 ms.
+// Partials are laid out [row][block]; row 0 holds t.t, row 1 + i V_i.t.
+__device__ inline void two_sum(double &hi, double &lo, double x) {
+    const double s = hi + x, z = s - hi;
+    lo += (hi - (s - z)) + (x - z);
+    hi = s;
+}
+// sum of one row of partials by a wave, in twice the working precision (as the host's
+// long double sums were at least)
+__device__ inline double row_sum(const double *__restrict__ row, int nblk, int lane) {
+    double hi = 0.0, lo = 0.0;
+    for (int b = lane; b < nblk; b += 64) two_sum(hi, lo, row[b]);
+    for (int o = 32; o > 0; o >>= 1) {
+        const double h2 = __shfl_xor(hi, o, 64), l2 = __shfl_xor(lo, o, 64);
+        two_sum(hi, lo, h2);
+        lo += l2;
+    }
+    return __shfl(hi + lo, 0, 64);  // one lane's rounding for all
+}
+// block sums of up to 4 per-thread values
+template <int N>
+__device__ inline void block_sums(double (&v)[N], double *red) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+        for (int o = 32; o > 0; o >>= 1) v[k] += __shfl_xor(v[k], o, 64);
+    __syncthreads();  // red free
+    if (lane == 0)
+#pragma unroll
+        for (int k = 0; k < N; ++k) red[wave * N + k] = v[k];
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < N; ++k) v[k] = (red[k] + red[N + k]) + (red[2 * N + k] + red[3 * N + k]);
+}
+
+// MODE 0: dots of t.  MODE 1: t = f u - r first, f = (r.u)/(u.u) from pin rows 1, 2.
+// MODE 2: t -= sum_i w_i (V_i.t) V_i first, the products from pin (w null: all 1); with
+// ptau, only when |t| (pin row 0) fell below a quarter of ptau's row 0, the
+// refinement test of jacobi.h:384-393.  Block b owns elements [b * chunk, (b+1) * chunk).
+template <int MODE>
+__global__ void __launch_bounds__(256) k_orth(const double *__restrict__ V, int64_t n, int64_t chunk, int m,
+                                              double *t, const double *u, const double *r,
+                                              const double *__restrict__ w, const double *__restrict__ pin,
+                                              const double *__restrict__ ptau, int self,
+                                              double *__restrict__ pout) {
+    extern __shared__ double coef[];  // m
+    __shared__ double red[16];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nblk = gridDim.x;
+    const int64_t lo = blockIdx.x * chunk, hi = min(n, lo + chunk);
+    if (MODE == 1) {
+        const double f = row_sum(pin + nblk, nblk, lane) / row_sum(pin + 2 * nblk, nblk, lane);
+        for (int64_t e = lo + threadIdx.x; e < hi; e += 256) t[e] = fma(f, u[e], -r[e]);
+    }
+    if (MODE == 2) {
+        if (ptau && sqrt(row_sum(pin, nblk, lane)) >= 0.25 * sqrt(row_sum(ptau, nblk, lane))) return;
+        for (int i = wave; i < m; i += 4) {
+            const double d = row_sum(pin + (int64_t)(i + 1) * nblk, nblk, lane);
+            if (lane == 0) coef[i] = w ? d * w[i] : d;
+        }
+        __syncthreads();
+        for (int64_t e = lo + threadIdx.x; e < hi; e += 256) {
+            double a = t[e];
+            for (int i = 0; i < m; ++i) a = fma(-coef[i], V[i * n + e], a);
+            t[e] = a;
+        }
+    }
+    // each thread reads back only elements it wrote itself
+    for (int p = self ? -1 : 0; p < m; p += 4) {
+        double acc[4] = {0, 0, 0, 0};
+        const int k = min(4, m - p);
+        for (int64_t e = lo + threadIdx.x; e < hi; e += 256) {
+            const double x = t[e];
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (q < k) acc[q] = fma(p + q < 0 ? x : V[(p + q) * n + e], x, acc[q]);
+        }
+        block_sums<4>(acc, red);
+        if (threadIdx.x < 4 && (int)threadIdx.x < k) {
+            const double s = threadIdx.x == 0 ? acc[0] : threadIdx.x == 1 ? acc[1] : threadIdx.x == 2 ? acc[2] : acc[3];
+            pout[(int64_t)(p + (int)threadIdx.x + (self ? 1 : 0)) * nblk + blockIdx.x] = s;
+        }
+    }
+}
+
+// t /= |t|: the norm from p2's row 0 when the second update ran (see k_orth), else p1's;
+// p0 null: from p1
+__global__ void __launch_bounds__(256) k_normalise(double *t, int64_t n, int nblk, const double *__restrict__ p0,
+                                                   const double *__restrict__ p1, const double *__restrict__ p2) {
+    const int lane = threadIdx.x & 63;
+    double s = row_sum(p1, nblk, lane);
+    if (p0 && !(sqrt(s) >= 0.25 * sqrt(row_sum(p0, nblk, lane)))) s = row_sum(p2, nblk, lane);
+    const double f = 1.0 / sqrt(s);
+    for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < n; e += (int64_t)gridDim.x * blockDim.x)
+        t[e] = f * t[e];
+}
+
+// u = sum c V, r = sum c VA - theta u, and the partials of r.r, r.u, u.u (to device and
+// pinned host memory): one pass over the two bases.  Bases beyond kCombMax vectors
+// take several launches: `first` starts the sums, `last` forms r.
+__global__ void __launch_bounds__(256) k_ritz(const RitzArgs c, int nv, const double *__restrict__ V,
+                                              const double *__restrict__ VA, int64_t n, double theta, int first,
+                                              int last, double *u, double *r, double *__restrict__ pdev,
+                                              double *__restrict__ phost) {
+    __shared__ double red[12];
+    double acc[3] = {0, 0, 0};
+    for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < n; e += (int64_t)gridDim.x * blockDim.x) {
+        double a = first ? 0.0 : u[e], b = first ? 0.0 : r[e];
+#pragma unroll 4
+        for (int j = 0; j < nv; ++j) {
+            a = fma(c.c[j], V[j * n + e], a);
+            b = fma(c.c[j], VA[j * n + e], b);
+        }
+        if (last) b = fma(-theta, a, b);
+        u[e] = a;
+        r[e] = b;
+        acc[0] = fma(b, b, acc[0]);
+        acc[1] = fma(b, a, acc[1]);
+        acc[2] = fma(a, a, acc[2]);
+    }
+    if (!last) return;
+    block_sums<3>(acc, red);
+    if (threadIdx.x == 0)
+        for (int k = 0; k < 3; ++k) {
+            pdev[k * gridDim.x + blockIdx.x] = acc[k];
+            phost[k * gridDim.x + blockIdx.x] = acc[k];
+        }
 }
 
 // ------------------------------------------------------------------ launchers
@@ -767,9 +903,34 @@ hipError_t launch_gemm(const GemmGroup *groups, const GemmTile *tiles, int ntile
                                              s);
 }
 
-hipError_t launch_multidot(const double *const *xs, const double *const *ys, int npairs, int64_t n, int nblocks,
-                           double *partial, hipStream_t s) {
-    hipLaunchKernelGGL(k_multidot, dim3(nblocks, npairs), dim3(256), 0, s, xs, ys, n, partial);
+hipError_t launch_multidot(const PairArgs &a, int npairs, int64_t n, int nblocks, double *partial, hipStream_t s) {
+    hipLaunchKernelGGL(k_multidot, dim3(nblocks, npairs), dim3(256), 0, s, a, n, partial);
+    return hipGetLastError();
+}
+hipError_t launch_orth(OrthMode mode, const double *V, int64_t n, int m, double *t, const double *u, const double *r,
+                       const double *w, const double *pin, const double *ptau, bool self, int nblocks, double *pout,
+                       hipStream_t s) {
+    const int64_t chunk = (n + nblocks - 1) / nblocks;
+    const dim3 g(nblocks), b(256);
+    const size_t lds = sizeof(double) * std::max(1, m);
+    if (mode == ORTH_DOTS)
+        hipLaunchKernelGGL((k_orth<0>), g, b, lds, s, V, n, chunk, m, t, u, r, w, pin, ptau, self, pout);
+    else if (mode == ORTH_CORRECTION)
+        hipLaunchKernelGGL((k_orth<1>), g, b, lds, s, V, n, chunk, m, t, u, r, w, pin, ptau, self, pout);
+    else
+        hipLaunchKernelGGL((k_orth<2>), g, b, lds, s, V, n, chunk, m, t, u, r, w, pin, ptau, self, pout);
+    return hipGetLastError();
+}
+hipError_t launch_normalise(double *t, int64_t n, int nblocks, const double *p0, const double *p1, const double *p2,
+                            hipStream_t s) {
+    const int nb = (int)std::max<int64_t>(1, std::min<int64_t>((n + 255) / 256, 1024));
+    hipLaunchKernelGGL(k_normalise, dim3(nb), dim3(256), 0, s, t, n, nblocks, p0, p1, p2);
+    return hipGetLastError();
+}
+hipError_t launch_ritz(const RitzArgs &c, int nv, const double *V, const double *VA, int64_t n, double theta,
+                       bool first, bool last, double *u, double *r, int nblocks, double *pdev, double *phost,
+                       hipStream_t s) {
+    hipLaunchKernelGGL(k_ritz, dim3(nblocks), dim3(256), 0, s, c, nv, V, VA, n, theta, first, last, u, r, pdev, phost);
     return hipGetLastError();
 }
 __global__ void __launch_bounds__(256) k_diag_scale(const double *x, const double *u, double f,
@@ -790,11 +951,10 @@ hipError_t launch_diag_scale(const double *x, const double *u, double f, const d
     return hipGetLastError();
 }
 
-hipError_t launch_lincomb(const double *const *vs, const double *coef, int nv, int64_t n, double beta, double *out,
-                          hipStream_t s) {
+hipError_t launch_lincomb(const CombArgs &a, int nv, int64_t n, double beta, double *out, hipStream_t s) {
     int nb = (int)std::min<int64_t>((n + 255) / 256, 4096);
     if (nb < 1) nb = 1;
-    hipLaunchKernelGGL(k_lincomb, dim3(nb), dim3(256), 0, s, vs, coef, nv, n, beta, out);
+    hipLaunchKernelGGL(k_lincomb, dim3(nb), dim3(256), 0, s, a, nv, n, beta, out);
     return hipGetLastError();
 }
 

@@ -41,14 +41,38 @@ hipError_t launch_gemm(const GemmGroup *groups, const GemmTile *tiles, int ntile
 hipError_t launch_gemm(const GemmGroup *groups, const GemmTile *tiles, int ntiles, const int *split_gids, int nsplit, int rblocks,
                        const float *A, const float *B, double *C, float *W, const RowMap *rowmap, int stage,
                        hipStream_t s, bool bf16x3 = false);
-hipError_t launch_multidot(const double *const *xs, const double *const *ys, int npairs, int64_t n, int nblocks,
-                           double *partial, hipStream_t s);
+// Davidson vector operations.  Vector pairs and coefficients are kernel arguments, at
+// most kCombMax per launch.
+constexpr int kCombMax = 48;
+struct PairArgs {
+    const double *x[kCombMax], *y[kCombMax];
+};
+struct CombArgs {
+    const double *v[kCombMax];
+    double c[kCombMax];
+};
+struct RitzArgs {
+    double c[kCombMax];
+};
+// partial[p * nblocks + block] of x_p . y_p (device or pinned host memory)
+hipError_t launch_multidot(const PairArgs &a, int npairs, int64_t n, int nblocks, double *partial, hipStream_t s);
+// one step of an orthonormalisation against V (m vectors, one after another); partials
+// are [row][block], row 0 t.t (when self), then V_i.t; see k_orth
+enum OrthMode { ORTH_DOTS = 0, ORTH_CORRECTION = 1, ORTH_UPDATE = 2 };
+hipError_t launch_orth(OrthMode mode, const double *V, int64_t n, int m, double *t, const double *u, const double *r,
+                       const double *w, const double *pin, const double *ptau, bool self, int nblocks, double *pout,
+                       hipStream_t s);
+hipError_t launch_normalise(double *t, int64_t n, int nblocks, const double *p0, const double *p1, const double *p2,
+                            hipStream_t s);
+// Ritz vector u, residual r and the partials of r.r, r.u, u.u; see k_ritz
+hipError_t launch_ritz(const RitzArgs &c, int nv, const double *V, const double *VA, int64_t n, double theta,
+                       bool first, bool last, double *u, double *r, int nblocks, double *pdev, double *phost,
+                       hipStream_t s);
 // out = (x - f u) / (theta - D), elementwise, leaving the elements where theta == D
 // undivided (MultDiagonal::mult_diag); out may alias x
 hipError_t launch_diag_scale(const double *x, const double *u, double f, const double *D, double theta, double *out,
                              int64_t n, hipStream_t s);
-hipError_t launch_lincomb(const double *const *vs, const double *coef, int nv, int64_t n, double beta, double *out,
-                          hipStream_t s);
+hipError_t launch_lincomb(const CombArgs &a, int nv, int64_t n, double beta, double *out, hipStream_t s);
 // two-site split: gather psi into the SVD working matrices (X must be zeroed
 // first) and the assembly of the two site tensors
 hipError_t launch_split_gather(const SplitSlab *slabs, int n, const double *psi, double *X, hipStream_t s);
