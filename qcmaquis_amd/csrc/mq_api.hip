@@ -118,16 +118,30 @@ void check(hipError_t e, const char *what) {
     if (e != hipSuccess) throw std::runtime_error(std::string(what) + ": " + hipGetErrorString(e));
 }
 
-// packs must cover the strips in order, each with 1..kPackStrips strips
+// packs must cover the strips and their elements in order
 void check_packs(const StripList &sl) {
-    const auto &p = sl.packs;
-    if (sl.strips.empty() && p.size() <= 1) return;
-    if (p.size() < 2 || p.front() != 0 || p.back() != (int)sl.strips.size())
-        throw std::runtime_error("strip packs do not cover the strip list");
-    for (size_t i = 0; i + 1 < p.size(); ++i)
-        if (p[i + 1] - p[i] < 1 || p[i + 1] - p[i] > kPackStrips) throw std::runtime_error("strip pack out of range");
+    int next = 0;
+    int64_t done = 0;  // elements of strip `next` covered by passes
+    for (auto &k : sl.packs) {
+        if (k.first != next || k.n < 1 || k.n > kPackStrips || next + k.n > (int)sl.strips.size())
+            throw std::runtime_error("strip pack out of range");
+        if (k.e0 == kPackWaves) {
+            if (k.n > 4 || done) throw std::runtime_error("strip pack too large");
+            next += k.n;
+        } else if (k.e0 < 0) {
+            int64_t el = 0;
+            for (int i = 0; i < k.n; ++i) el += (int64_t)sl.strips[next + i].rows * sl.strips[next + i].cols;
+            if (el > kPackElems || done) throw std::runtime_error("strip pack too large");
+            next += k.n;
+        } else {
+            if (k.n != 1 || k.e0 != done) throw std::runtime_error("strip passes out of order");
+            done += kPassElems;
+            if (done >= (int64_t)sl.strips[next].rows * sl.strips[next].cols) ++next, done = 0;
+        }
+    }
+    if (next != (int)sl.strips.size()) throw std::runtime_error("strip packs do not cover the strip list");
 }
-int npacks(const StripList &sl) { return sl.packs.empty() ? 0 : (int)sl.packs.size() - 1; }
+int npacks(const StripList &sl) { return (int)sl.packs.size(); }
 
 }  // namespace
 
@@ -137,7 +151,7 @@ struct mq_plan {
     DevArray<Copy2D> arrL, arrR, reshape, scatter;
     DevArray<Strip> strips, cstrips;
     DevArray<Src> srcs, csrcs;
-    DevArray<int> packs, cpacks;  // strip packs of wapply / combL
+    DevArray<Pack> packs, cpacks;  // strip packs of wapply / combL
     DevGemm g1, g2;
     DevArray<double> la, rb, prp, t, c, tmp, ws;
     double w_src_el = 0, w_dst_el = 0;  // W-application source / destination elements

@@ -39,87 +39,103 @@ __global__ void __launch_bounds__(256) k_to_f32(const double *__restrict__ src, 
 
 // ------------------------------------------------------------------ W application
 // dst strip = sum_s coef_s * src_s, summed in task order (deterministic, no
-// atomics).  Each thread owns WU elements of a pass, so every source issues
-// WU independent loads before they are accumulated; element e of the strip
-// is (i, j) = (e mod rows, e / rows), the quotient taken from a float
-// reciprocal and corrected (exact for strips below 2^24 elements).
+// atomics).  Element e of a strip is (i, j) = (e mod rows, e / rows), the quotient taken
+// from a float reciprocal and corrected (exact for strips below 2^24 elements).
 constexpr int WU = 4;
 
-// One workgroup per pack of consecutive strips (see StripList): a pack of one
-// large strip runs the strip with all threads; a pack of several small strips
-// runs their elements as one index range, each element finding its strip with a
-// binary search over the pack's element offsets in LDS.
-// A large strip gives each thread WS = 8 elements per pass, so that a wave has
-// 2 KB (FP32) or 4 KB (FP64) of loads in flight per source: the W application is
-// bound by the bytes in flight per wave more than by instructions (measured at
-// the L=24 centre: FP32 1.06 -> 1.00 ms from 4 to 8 elements, FP64 1.77 -> 1.72 ms;
-// 16 FP32 elements gained nothing more).
-template <class T>
-constexpr int strip_units() {
-    return 8;
-}
-template <class T>
-__device__ __forceinline__ void wapply_strip(const Strip &st, const Src *__restrict__ srcs, const T *__restrict__ src,
-                                             T *__restrict__ C) {
-    constexpr int WS = strip_units<T>();
+// One pass over a large strip: each thread owns WS = 8 elements, so that a wave has
+// 2 KB (FP32) or 4 KB (FP64) of loads in flight per source: the kernel is bound by the
+// bytes in flight per wave more than by instructions (L=24 centre: FP32 1.06 -> 1.00 ms
+// from 4 to 8 elements, FP64 1.77 -> 1.72 ms; 16 FP32 elements gained nothing more).
+// The strips of a fused-row combination sum hundreds of sources, a serial chain: one
+// workgroup per pass instead of per strip spreads them over more CUs, and the next
+// source record is read before the current one is used.
+constexpr int WS = kPassElems / 256;
+// (NT threads, this one's number t, elements from e0 on)
+template <class T, int NT>
+__device__ __forceinline__ void wapply_pass(const Strip &st, int e0, int t, const Src *__restrict__ srcs,
+                                            const T *__restrict__ src, T *__restrict__ C) {
     const int rows = st.rows, n = st.rows * st.cols;
     const float inv = 1.0f / (float)max(rows, 1);
-    for (int base = 0; base < n; base += 256 * WS) {
-        int ii[WS], jj[WS];
-        T acc[WS];
+    int ii[WS], jj[WS];
+    T acc[WS];
 #pragma unroll
-        for (int u = 0; u < WS; ++u) {
-            const int e = base + threadIdx.x + 256 * u;
-            int j = (int)((float)e * inv);
-            if (j * rows > e) --j;
-            else if ((j + 1) * rows <= e) ++j;
-            ii[u] = e - j * rows;
-            jj[u] = e < n ? j : -1;
-            acc[u] = 0;
-        }
-        for (int s = st.s0; s < st.s1; ++s) {
-            const Src sr = srcs[s];
-            const T c = (T)sr.coef;
-            T v[WS];
-#pragma unroll
-            for (int u = 0; u < WS; ++u) v[u] = jj[u] >= 0 ? src[sr.off + ii[u] + (int64_t)jj[u] * sr.ld] : (T)0;
-#pragma unroll
-            for (int u = 0; u < WS; ++u) acc[u] += c * v[u];
-        }
-#pragma unroll
-        for (int u = 0; u < WS; ++u)
-            if (jj[u] >= 0) C[st.dst + ii[u] + (int64_t)jj[u] * st.ldd] = acc[u];
+    for (int u = 0; u < WS; ++u) {
+        const int e = e0 + t + NT * u;
+        int j = (int)((float)e * inv);
+        if (j * rows > e) --j;
+        else if ((j + 1) * rows <= e) ++j;
+        ii[u] = e - j * rows;
+        jj[u] = e < n ? j : -1;
+        acc[u] = 0;
     }
+    Src nx{};
+    if (st.s0 < st.s1) nx = srcs[st.s0];
+    for (int s = st.s0; s < st.s1; ++s) {
+        const Src sr = nx;
+        nx = srcs[min(s + 1, st.s1 - 1)];
+        const T c = (T)sr.coef;
+        T v[WS];
+#pragma unroll
+        for (int u = 0; u < WS; ++u) v[u] = jj[u] >= 0 ? src[sr.off + ii[u] + (int64_t)jj[u] * sr.ld] : (T)0;
+#pragma unroll
+        for (int u = 0; u < WS; ++u) acc[u] += c * v[u];
+    }
+#pragma unroll
+    for (int u = 0; u < WS; ++u)
+        if (jj[u] >= 0) C[st.dst + ii[u] + (int64_t)jj[u] * st.ldd] = acc[u];
 }
 
 static_assert(kPackElems <= 256 * WU, "a pack of small strips is run in one pass");
+static_assert(kPackStrips == 64, "one lane per strip of a pack");
 
+// One workgroup per pack (see StripList).  A pack of small strips runs their elements as
+// one index range, each element finding its strip with a binary search over the pack's
+// element offsets in LDS (a wave scan: one lane summing them took 2 us of every
+// workgroup's life, which at L=8 m=64 is all that the launch lasts).
 // nvec vectors share one task list: vector v reads src + v * sstride and writes
 // C + v * dstride (the batched sigma), so the strip and source records are read
 // once per workgroup for all of them.
 // (MULTI false: one vector, compiled without the vector loop.)
 template <int STAGE, class T, bool MULTI>
-__global__ void __launch_bounds__(256) k_wapply(const Strip *__restrict__ strips, const int *__restrict__ packs,
+__global__ void __launch_bounds__(256) k_wapply(const Strip *__restrict__ strips, const Pack *__restrict__ packs,
                                                 const Src *__restrict__ srcs, const T *__restrict__ src,
                                                 T *__restrict__ C, int nvec_arg, int64_t sstride, int64_t dstride) {
     const int nvec = MULTI ? nvec_arg : 1;
-    const int p0 = packs[blockIdx.x], ns = packs[blockIdx.x + 1] - p0;
-    if (ns == 1) {
+    const Pack pk = packs[blockIdx.x];
+    const int p0 = pk.first, ns = pk.n;
+    if (pk.e0 >= 0) {
         const Strip st = strips[p0];
-        for (int v = 0; v < nvec; ++v) wapply_strip<T>(st, srcs, src + v * sstride, C + v * dstride);
+        for (int v = 0; v < nvec; ++v)
+            wapply_pass<T, 256>(st, pk.e0, threadIdx.x, srcs, src + v * sstride, C + v * dstride);
+        return;
+    }
+    if (pk.e0 == kPackWaves) {
+        const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        if (w >= ns) return;
+        const Strip st = strips[p0 + w];
+        for (int v = 0; v < nvec; ++v)
+            for (int e = 0; e < st.rows * st.cols; e += 64 * WS)
+                wapply_pass<T, 64>(st, e, threadIdx.x & 63, srcs, src + v * sstride, C + v * dstride);
         return;
     }
     __shared__ Strip sst[kPackStrips];
     __shared__ int pre[kPackStrips + 1];
-    if ((int)threadIdx.x < ns) sst[threadIdx.x] = strips[p0 + threadIdx.x];
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int acc = 0;
-        for (int k = 0; k < ns; ++k) {
-            pre[k] = acc;
-            acc += sst[k].rows * sst[k].cols;
+    if (threadIdx.x < 64) {
+        int el = 0;
+        if ((int)threadIdx.x < ns) {
+            const Strip st = strips[p0 + threadIdx.x];
+            sst[threadIdx.x] = st;
+            el = st.rows * st.cols;
         }
-        pre[ns] = acc;
+        int sum = el;  // inclusive scan over the wave
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int x = __shfl_up(sum, o, 64);
+            if ((int)threadIdx.x >= o) sum += x;
+        }
+        pre[threadIdx.x + 1] = sum;
+        if (threadIdx.x == 0) pre[0] = 0;
     }
     __syncthreads();
     const int total = pre[ns];  // at most kPackElems = 256 * WU: one pass
@@ -811,7 +827,7 @@ hipError_t launch_to_f32(const double *src, float *dst, int64_t n, hipStream_t s
 }
 
 template <class T, bool MULTI>
-static void wapply_stage(const Strip *strips, const int *packs, int npacks, const Src *srcs, const T *src, T *C,
+static void wapply_stage(const Strip *strips, const Pack *packs, int npacks, const Src *srcs, const T *src, T *C,
                          int stage, hipStream_t s, int nvec, int64_t ss, int64_t ds) {
     const dim3 g(npacks), b(256);
     switch (stage) {
@@ -830,7 +846,7 @@ static void wapply_stage(const Strip *strips, const int *packs, int npacks, cons
     }
 }
 template <class T>
-static hipError_t wapply_launch(const Strip *strips, const int *packs, int npacks, const Src *srcs, const T *src,
+static hipError_t wapply_launch(const Strip *strips, const Pack *packs, int npacks, const Src *srcs, const T *src,
                                 T *C, int stage, hipStream_t s, int nvec, int64_t ss, int64_t ds) {
     if (npacks == 0 || nvec < 1) return hipSuccess;
     if (nvec == 1)
@@ -839,11 +855,11 @@ static hipError_t wapply_launch(const Strip *strips, const int *packs, int npack
         wapply_stage<T, true>(strips, packs, npacks, srcs, src, C, stage, s, nvec, ss, ds);
     return hipGetLastError();
 }
-hipError_t launch_wapply(const Strip *strips, const int *packs, int npacks, const Src *srcs, const double *T,
+hipError_t launch_wapply(const Strip *strips, const Pack *packs, int npacks, const Src *srcs, const double *T,
                          double *C, int stage, hipStream_t s, int nvec, int64_t src_stride, int64_t dst_stride) {
     return wapply_launch<double>(strips, packs, npacks, srcs, T, C, stage, s, nvec, src_stride, dst_stride);
 }
-hipError_t launch_wapply(const Strip *strips, const int *packs, int npacks, const Src *srcs, const float *T, float *C,
+hipError_t launch_wapply(const Strip *strips, const Pack *packs, int npacks, const Src *srcs, const float *T, float *C,
                          int stage, hipStream_t s, int nvec, int64_t src_stride, int64_t dst_stride) {
     return wapply_launch<float>(strips, packs, npacks, srcs, T, C, stage, s, nvec, src_stride, dst_stride);
 }

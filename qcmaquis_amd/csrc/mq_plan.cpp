@@ -16,6 +16,7 @@
 #include <atomic>
 #include <cstdlib>
 #include <exception>
+#include <map>
 #include <mutex>
 #include <new>
 #include <thread>
@@ -400,33 +401,61 @@ PRP prp_layout(const Site &s, std::vector<Copy2D> &tasks) {
 //     sum_b1 w_b1 T[b1](slice) = (sum_b1 w_b1 L[b1])^T psi(slice),  w = e.coeff * scale.
 // Quantum-chemistry MPOs have a few columns (complementary operators) with
 // hundreds of terms but only a few hundred distinct positions; those columns
-// are "fused": each position becomes a fused group whose boundary rows are
-// combined once per boundary binding, and whose T slice is one small GEMM
-// per sigma.  The other columns keep their terms ("direct").
+// are "fused".  A fused column's W application is folded into the left
+// boundary: for the output state (phys block, state, lb) and the input state
+// (phys block, state, lk) the combined block
+//     F(lb, lk) = sum_b1 (sum of the positions' coupling * w_b1) L[b1](lb, lk)
+// is built once per boundary binding, and one GEMM whose K runs over all input states
+// of a right charge writes the column's C rows (through T) in one product.  The
+// positions used to have a T slice each, summed by the W application: at the L=24
+// m=512 centre 289 M of T's 501 M elements, written and read back once per sigma.
+// The other columns keep their terms ("direct").
 struct CTerm {
     int row;  // MPO row b1
     int op;
     double scale;
     int spin;  // 2S of the left MPO bond (a)
 };
-struct FBlk {  // one (lb, lk) block of a fused group
-    int lb, lk, ar, al;
-    int64_t lf;  // LA-arena offset of its first combined row (column 0)
-    int64_t tf;  // T-arena offset of its T block (stored contiguously, leading dimension |lb|)
-    int ld;      // rows of the fused LA panel (its leading dimension)
+struct FMem {  // one operator entry of MPO row b1
+    int b1;
+    int cls;  // index into FIn::cls
+    double w;
 };
-struct FGroup {
-    int b2, pin, pout, row, col, rspin, cspin, k, a;
-    std::vector<std::pair<int, double>> mem;  // (b1, weight)
-    std::vector<FBlk> blk;
+struct FCls {  // spin case of the entry (case_of), 2S of its operator, 2S of its left bond
+    int cs, k, a;
+};
+struct FIn {  // input state `row` of physical block pin
+    int pin, row;
+    std::vector<FCls> cls;
+    std::vector<FMem> mem;  // ascending b1
+};
+struct FChunk {  // F(lb, lk) of input `in`
+    int in, lk;
+    int nsrc;
+};
+struct FRow {  // the |lb| rows of one output (lb, al) and one right charge ar
+    int lb, al, ar;
+    int panel, row;
+    int64_t tf;  // T-arena offset of its T block (stored contiguously, leading dimension |lb|)
+    std::vector<FChunk> chunk;
+};
+struct FOut {  // output state `col` of physical block pout in column b2
+    int b2, pout, col;
+    std::vector<FIn> in;
+    std::vector<FRow> rows;
 };
 struct ColProg {
     std::vector<std::vector<CTerm>> col;  // [b2] direct terms
-    std::vector<std::vector<int>> fcol;   // [b2] fused group ids
-    std::vector<FGroup> fg;
-    std::vector<char> direct, member;     // [b1] row has direct terms / feeds a fused group
+    std::vector<std::vector<int>> fcol;   // [b2] ids of its fused outputs
+    std::vector<FOut> fo;
+    std::vector<char> direct, member;     // [b1] row has direct terms / feeds a fused column
 };
 
+// Besides many entries per position, many entries per output state make a column worth
+// fusing: they are the serial chain of sources that every element of its C rows sums in
+// the W application.  2 * ratio (8 by default) per output state: at L=8 and L=16 this
+// takes the longest chain from 30 and 47 sources to 5 (W application 28 -> 10 and 56 -> 23
+// us); at L=24 m=512 it fuses the same columns as the first rule.
 // fuse.mode: 0 never, 1 when a column's entries are at least fuse.ratio times its
 // distinct positions and number at least fuse.min_entries, 2 every non-empty
 // column (used by tests to exercise fused groups on small systems)
@@ -441,8 +470,8 @@ ColProg column_program(const Site &s, bool skip_rskip_cols, FuseRule fuse) {
         int b1;
         double w;
     };
-    // per column, in parallel: its direct terms (cp.col[b2]) or its fused groups
-    std::vector<std::vector<FGroup>> groups(s.W.cols);
+    // per column, in parallel: its direct terms (cp.col[b2]) or its fused outputs
+    std::vector<std::vector<FOut>> outs(s.W.cols);
     std::vector<char> fused_col(s.W.cols, 0);
     parallel_for(
         s.W.cols,
@@ -458,58 +487,64 @@ ColProg column_program(const Site &s, bool skip_rskip_cols, FuseRule fuse) {
                             if (ob.pin > 255 || ob.pout > 255 || e.row > 255 || e.col > 255 || e.rspin > 3 ||
                                 e.cspin > 3 || op.spin > 127 || s.W.lspin[b1] > 127)
                                 throw std::runtime_error("operator entry out of the fused-key range");
-                            uint64_t key = ((uint64_t)ob.pin << 56) | ((uint64_t)ob.pout << 48) |
-                                           ((uint64_t)e.row << 40) | ((uint64_t)e.col << 32) |
+                            uint64_t key = ((uint64_t)ob.pout << 56) | ((uint64_t)e.col << 48) |
+                                           ((uint64_t)ob.pin << 40) | ((uint64_t)e.row << 32) |
                                            ((uint64_t)e.rspin << 30) | ((uint64_t)e.cspin << 28) |
                                            ((uint64_t)op.spin << 21) | ((uint64_t)s.W.lspin[b1] << 14);
                             ents.push_back({key, b1, e.coeff * term.scale});
                         }
                 }
             std::stable_sort(ents.begin(), ents.end(), [](const E &x, const E &y) { return x.key < y.key; });
-            size_t ngroups = 0;
-            for (size_t i = 0; i < ents.size(); ++i)
+            size_t ngroups = 0, nouts = 0;
+            for (size_t i = 0; i < ents.size(); ++i) {
                 if (i == 0 || ents[i].key != ents[i - 1].key) ++ngroups;
+                if (i == 0 || (ents[i].key >> 48) != (ents[i - 1].key >> 48)) ++nouts;
+            }
             bool fused = (fuse.mode == 2 && !ents.empty()) ||
-                         (fuse.mode == 1 && !ents.empty() && ents.size() >= (size_t)fuse.min_entries &&
-                          ents.size() >= (size_t)fuse.ratio * ngroups);
+                         (fuse.mode == 1 && ents.size() >= (size_t)fuse.min_entries &&
+                          (ents.size() >= (size_t)fuse.ratio * ngroups ||
+                           ents.size() >= (size_t)2 * fuse.ratio * nouts));
             if (!fused) {
                 for (int b1 : s.W.col_b1[b2])
                     for (auto &term : s.W.terms(b1, b2)) cp.col[b2].push_back({b1, term.op, term.scale, s.W.lspin[b1]});
                 return;
             }
             fused_col[b2] = 1;
-            size_t i = 0;
-            while (i < ents.size()) {
+            for (size_t i = 0; i < ents.size();) {
                 size_t j = i;
-                while (j < ents.size() && ents[j].key == ents[i].key) ++j;
-                uint64_t k = ents[i].key;
-                FGroup g;
-                g.b2 = b2;
-                g.pin = (int)(k >> 56);
-                g.pout = (int)((k >> 48) & 255);
-                g.row = (int)((k >> 40) & 255);
-                g.col = (int)((k >> 32) & 255);
-                g.rspin = (int)((k >> 30) & 3);
-                g.cspin = (int)((k >> 28) & 3);
-                g.k = (int)((k >> 21) & 127);
-                g.a = (int)((k >> 14) & 127);
-                for (size_t q = i; q < j; ++q) g.mem.push_back({ents[q].b1, ents[q].w});
-                groups[b2].push_back(std::move(g));
+                while (j < ents.size() && (ents[j].key >> 32) == (ents[i].key >> 32)) ++j;
+                const uint64_t k = ents[i].key;
+                const int pout = (int)(k >> 56), col = (int)((k >> 48) & 255);
+                if (outs[b2].empty() || outs[b2].back().pout != pout || outs[b2].back().col != col)
+                    outs[b2].push_back({b2, pout, col, {}, {}});
+                FIn in{(int)((k >> 40) & 255), (int)((k >> 32) & 255), {}, {}};
+                in.mem.reserve(j - i);
+                for (size_t q = i; q < j; ++q) {
+                    if (q == i || ents[q].key != ents[q - 1].key) {
+                        const uint64_t c = ents[q].key;
+                        in.cls.push_back({case_of((int)((c >> 30) & 3), (int)((c >> 28) & 3)), (int)((c >> 21) & 127),
+                                          (int)((c >> 14) & 127)});
+                    }
+                    in.mem.push_back({ents[q].b1, (int)in.cls.size() - 1, ents[q].w});
+                }
+                std::stable_sort(in.mem.begin(), in.mem.end(), [](const FMem &x, const FMem &y) { return x.b1 < y.b1; });
+                outs[b2].back().in.push_back(std::move(in));
                 i = j;
             }
         },
         8, 1);
-    // in column order: the rows with direct terms, the group ids
+    // in column order: the rows with direct terms, the output ids
     for (int b2 = 0; b2 < s.W.cols; ++b2) {
         if (skip_rskip_cols && s.W.rskip(b2)) continue;
         if (!fused_col[b2]) {
             for (int b1 : s.W.col_b1[b2]) cp.direct[b1] = 1;
             continue;
         }
-        for (auto &g : groups[b2]) {
-            for (auto &m : g.mem) cp.member[m.first] = 1;
-            cp.fcol[b2].push_back((int)cp.fg.size());
-            cp.fg.push_back(std::move(g));
+        for (auto &o : outs[b2]) {
+            for (auto &in : o.in)
+                for (auto &m : in.mem) cp.member[m.b1] = 1;
+            cp.fcol[b2].push_back((int)cp.fo.size());
+            cp.fo.push_back(std::move(o));
         }
     }
     return cp;
@@ -534,12 +569,12 @@ struct TLay {
 // for its FLOP count).  Otherwise:
 //   LA arena = [LA_lk panels: direct rows, then staged rows | fused panels]
 //   T arena  = [T_lk panels (direct rows)                   | fused T panels]
-// A fused panel, keyed (lk, input block, input state), stacks the (group, lb)
-// rows of every fused group at that input; its T GEMM reads only the psi
-// columns of that input state (one right charge ar).  The combination strips
-// (comb) build the fused panels from the arranged rows.
-TLay t_layout(const Site &s, const BLayout &L, const PRP &prp, ColProg *cp, std::vector<Copy2D> *arr,
-              StripList *comb, GemmList *g1, int tm, int tn, int kc) {
+// A fused panel, keyed (ar, list of (input state, lk) chunks), stacks the rows of every
+// fused output with those chunks; its K runs over the chunks, and its B operand is
+// psi's rows of those chunks, packed into the psi arena by the reshape.  The
+// combination strips (comb) build the panels from the arranged rows.
+TLay t_layout(const Site &s, const BLayout &L, PRP &prp, ColProg *cp, std::vector<Copy2D> *arr,
+              std::vector<Copy2D> *reshape, StripList *comb, GemmList *g1, int tm, int tn, int kc) {
     struct A {
         int lb, lk;
         const BBlk *blk;
@@ -644,160 +679,202 @@ TLay t_layout(const Site &s, const BLayout &L, const PRP &prp, ColProg *cp, std:
             add_gemm(*g1, g, tm, tn, kc);
         }
     }
-    if (!cp || cp->fg.empty()) return t;
+    if (!cp || cp->fo.empty()) return t;
 
-    // ---- fused groups: blocks, panels, combination strips, T GEMMs
-    // Per-group work runs on a thread pool; every order-dependent step (panel and
-    // row assignment, source offsets) is sequential in group order, so the plan
+    // ---- fused columns: rows, panels, combination strips, GEMMs
+    // Per-output work runs on a thread pool; every order-dependent step (panel and
+    // row assignment, source offsets) is sequential in output order, so the plan
     // does not depend on the thread count.
     struct Panel {
-        int lk, pin, row, ar, rows = 0;
-        int64_t lf = 0, tf = 0;
+        int ar, K = 0, rows = 0;
+        int64_t lf = 0, tf = 0, pb = 0;         // LA, T and psi arena offsets
+        std::vector<std::array<int, 3>> chunk;  // (pin, row, lk)
         std::vector<std::pair<int, int>> blocks;  // (first row, rows) in row order
     };
-    struct Cand {
-        int lk, lb, ar, al;
-    };
     const int nl = s.nl;
-    const int ng = (int)cp->fg.size();
-    // 1. (parallel) union of the members' (lb, lk) blocks, in (lk, lb) order, kept when
-    //    the charges and spins let the block contribute
-    std::vector<std::vector<Cand>> cand(ng);
-    parallel_for(ng, [&](int gi) {
-        thread_local std::vector<char> mark;
-        mark.assign((size_t)nl * nl, 0);
-        const FGroup &g = cp->fg[gi];
-        const int ap = s.W.rspin[g.b2];
-        for (auto &m : g.mem)
-            for (auto &a : blk[m.first]) mark[(size_t)a.lk * nl + a.lb] = 1;
-        for (int lk = 0; lk < nl; ++lk)
+    const int ng = (int)cp->fo.size();
+    // coupling of class c of input `in` at (lk, lb); zero where the charges or spins do not
+    // let the block contribute
+    auto factor = [&](const FOut &o, const FIn &in, const FCls &c, int lk, int lb, int ar, int al) {
+        if (!s.su2) return 1.0;
+        const int ap = s.W.rspin[o.b2];
+        const int i = spin2(s.left.q[lb]), j = spin2(s.left.q[lk]);
+        const int jp = spin2(s.right.q[ar]), ip = spin2(s.right.q[al]);
+        if (!tri(jp, ap, ip)) return 0.0;
+        return coupling(j, std::abs(j - jp), jp, c.a, c.k, ap, i, std::abs(i - ip), ip)[c.cs];
+    };
+    // right charges of (input, lk) and (output, lb), -1 where psi or sigma has none
+    auto right_in = [&](const FIn &in, int lk) {
+        return s.pbr_sz_l[lk] == 0 ? -1 : s.lp_r[(size_t)lk * s.np + in.pin];
+    };
+    auto right_out = [&](const FOut &o, int lb) {
+        const int al = s.lp_r[(size_t)lb * s.np + o.pout];
+        return al >= 0 && s.x_of_r[al] >= 0 ? al : -1;
+    };
+    // f(in index, block, coefficient) for every source of output o: each L block of each
+    // member row, the entries of one row summed; blocks whose every coupling vanishes
+    // are left out
+    auto for_sources = [&](const FOut &o, auto &&f) {
+        thread_local std::vector<double> tab;  // [class][lk][lb]
+        thread_local std::vector<char> have;
+        for (size_t q = 0; q < o.in.size(); ++q) {
+            const FIn &in = o.in[q];
+            tab.assign(in.cls.size() * nl * nl, 0.0);
+            have.assign(in.cls.size() * nl * nl, 0);
+            for (size_t m0 = 0; m0 < in.mem.size();) {
+                size_t m1 = m0;
+                while (m1 < in.mem.size() && in.mem[m1].b1 == in.mem[m0].b1) ++m1;
+                for (auto &a : blk[in.mem[m0].b1]) {
+                    const int ar = right_in(in, a.lk), al = right_out(o, a.lb);
+                    if (ar < 0 || al < 0) continue;
+                    double c = 0.0;
+                    bool any = false;
+                    for (size_t m = m0; m < m1; ++m) {
+                        const size_t at = ((size_t)in.mem[m].cls * nl + a.lk) * nl + a.lb;
+                        if (!have[at]) {
+                            tab[at] = factor(o, in, in.cls[in.mem[m].cls], a.lk, a.lb, ar, al);
+                            have[at] = 1;
+                        }
+                        any = any || tab[at] != 0.0;
+                        c += in.mem[m].w * tab[at];
+                    }
+                    if (any) f((int)q, a, c);
+                }
+                m0 = m1;
+            }
+        }
+    };
+    // 1. (parallel) the rows of each output and their chunks, with source counts
+    parallel_for(
+        ng,
+        [&](int gi) {
+            FOut &o = cp->fo[gi];
+            thread_local std::vector<int> cnt;  // [lb][in][lk]
+            const size_t ni = o.in.size();
+            cnt.assign(ni * nl * nl, 0);
+            for_sources(o, [&](int q, const A &a, double) { ++cnt[((size_t)a.lb * ni + q) * nl + a.lk]; });
             for (int lb = 0; lb < nl; ++lb) {
-                if (!mark[(size_t)lk * nl + lb]) continue;
-                int ar = s.lp_r[(size_t)lk * s.np + g.pin];
-                if (ar < 0 || s.pbr_sz_l[lk] == 0) continue;
-                int al = s.lp_r[(size_t)lb * s.np + g.pout];
-                if (al < 0 || s.x_of_r[al] < 0) continue;  // out_left_i
-                if (s.su2 && !tri(spin2(s.right.q[ar]), ap, spin2(s.right.q[al]))) continue;
-                cand[gi].push_back({lk, lb, ar, al});
+                const int al = right_out(o, lb);
+                if (al < 0) continue;
+                const size_t r0 = o.rows.size();
+                for (size_t q = 0; q < ni; ++q)
+                    for (int lk = 0; lk < nl; ++lk) {
+                        const int n = cnt[((size_t)lb * ni + q) * nl + lk];
+                        if (n == 0) continue;
+                        const int ar = right_in(o.in[q], lk);
+                        size_t r = r0;
+                        while (r < o.rows.size() && o.rows[r].ar != ar) ++r;
+                        if (r == o.rows.size()) o.rows.push_back({lb, al, ar, 0, 0, 0, {}});
+                        o.rows[r].chunk.push_back({(int)q, lk, n});
+                    }
             }
-    });
-    // 2. (sequential) panels keyed by (lk, input block, input state < 256), rows in group order
-    const int nrow_states = 256;
-    std::vector<int> panel_id((size_t)nl * s.np * nrow_states, -1);
+        },
+        4, 1);
+    // 2. (sequential) panels keyed by (ar, chunks), rows in output order
+    std::map<std::vector<int>, int> panel_id;
     std::vector<Panel> panels;
-    std::vector<std::vector<std::pair<int, int>>> fb_panel(ng);  // per group block: (panel, row)
-    for (int gi = 0; gi < ng; ++gi) {
-        FGroup &g = cp->fg[gi];
-        g.blk.reserve(cand[gi].size());
-        fb_panel[gi].reserve(cand[gi].size());
-        for (auto &c : cand[gi]) {
-            int &pid = panel_id[((size_t)c.lk * s.np + g.pin) * nrow_states + g.row];
-            if (pid < 0) {
-                pid = (int)panels.size();
+    for (auto &o : cp->fo)
+        for (auto &r : o.rows) {
+            std::vector<int> key{r.ar};
+            for (auto &c : r.chunk) {
+                key.push_back(o.in[c.in].pin * 256 + o.in[c.in].row);
+                key.push_back(c.lk);
+            }
+            auto it = panel_id.emplace(key, (int)panels.size());
+            if (it.second) {
                 Panel pn;
-                pn.lk = c.lk;
-                pn.pin = g.pin;
-                pn.row = g.row;
-                pn.ar = c.ar;
-                panels.push_back(pn);
+                pn.ar = r.ar;
+                for (auto &c : r.chunk) {
+                    pn.chunk.push_back({o.in[c.in].pin, o.in[c.in].row, c.lk});
+                    pn.K += s.lsize(c.lk);
+                }
+                panels.push_back(std::move(pn));
             }
-            g.blk.push_back({c.lb, c.lk, c.ar, c.al, 0, 0, 0});
-            fb_panel[gi].push_back({pid, panels[pid].rows});
-            panels[pid].blocks.push_back({panels[pid].rows, s.lsize(c.lb)});
-            panels[pid].rows += s.lsize(c.lb);
+            r.panel = it.first->second;
+            Panel &pn = panels[r.panel];
+            r.row = pn.rows;
+            pn.blocks.push_back({pn.rows, s.lsize(r.lb)});
+            pn.rows += s.lsize(r.lb);
         }
-    }
     for (auto &pn : panels) {
+        const int rsz = s.rsize(pn.ar);
         pn.lf = t.la_total;
-        t.la_total += (int64_t)pn.rows * s.lsize(pn.lk);
+        t.la_total += (int64_t)pn.rows * pn.K;
         pn.tf = t.t_total;
-        t.t_total += (int64_t)pn.rows * s.rsize(pn.ar);
-    }
-    // 3. (parallel) block offsets and, per block, the number of member sources
-    std::vector<std::vector<int>> cnt(ng);
-    parallel_for(ng, [&](int gi) {
-        FGroup &g = cp->fg[gi];
-        const size_t nb = g.blk.size();
-        for (size_t k = 0; k < nb; ++k) {
-            FBlk &fb = g.blk[k];
-            const Panel &pn = panels[fb_panel[gi][k].first];
-            int row = fb_panel[gi][k].second;
-            fb.lf = pn.lf + row;
-            fb.tf = pn.tf + (int64_t)row * s.rsize(pn.ar);
-            fb.ld = pn.rows;
+        t.t_total += (int64_t)pn.rows * rsz;
+        if (!reshape) continue;
+        // psi's rows of the panel's chunks, one under the other (K x |ar|)
+        const VBlk &xb = s.X.blk[s.x_of_r[pn.ar]];
+        pn.pb = prp.total;
+        int k = 0;
+        for (auto &c : pn.chunk) {
+            const int ld = s.lsize(c[2]);
+            reshape->push_back(mk_copy(pn.pb + k, xb.off + s.pbl[(size_t)c[0] * nl + c[2]] + c[1] * ld, ld, rsz, pn.K,
+                                       xb.rows, false, 1.0));
+            k += ld;
         }
-        if (!comb) return;
-        thread_local std::vector<int> slot;
-        slot.assign((size_t)nl * nl, -1);
-        for (size_t k = 0; k < nb; ++k) slot[(size_t)g.blk[k].lk * nl + g.blk[k].lb] = (int)k;
-        cnt[gi].assign(nb, 0);
-        for (auto &m : g.mem)
-            for (auto &a : blk[m.first]) {
-                int k = slot[(size_t)a.lk * nl + a.lb];
-                if (k >= 0) ++cnt[gi][k];
-            }
-    });
-    std::vector<uint64_t> comb_key;  // (lk, lb): strips reading one LA_lk row range run together
+        prp.total += (int64_t)pn.K * rsz;
+    }
+    for (auto &o : cp->fo)
+        for (auto &r : o.rows) r.tf = panels[r.panel].tf + (int64_t)r.row * s.rsize(r.ar);
     if (comb) {
-        // 4. strips and source ranges in group order: offsets by prefix sums, then
-        //    (parallel) each group's strips
+        // 3. strips and source ranges in output order: offsets by prefix sums
         std::vector<int> gbase(ng + 1, (int)comb->srcs.size());
         std::vector<size_t> sbase(ng + 1, comb->strips.size());
         for (int gi = 0; gi < ng; ++gi) {
             int64_t nsrc = 0;
-            for (int c : cnt[gi]) nsrc += c;
+            size_t nst = 0;
+            for (auto &r : cp->fo[gi].rows) {
+                for (auto &c : r.chunk) nsrc += c.nsrc;
+                nst += r.chunk.size();
+            }
             if (gbase[gi] + nsrc > INT32_MAX) throw std::runtime_error("fused-row combination: too many sources");
             gbase[gi + 1] = gbase[gi] + (int)nsrc;
-            sbase[gi + 1] = sbase[gi] + cp->fg[gi].blk.size();
+            sbase[gi + 1] = sbase[gi] + nst;
         }
+        const size_t s0 = sbase[0];
         comb->strips.resize(sbase[ng]);
-        comb_key.resize(sbase[ng] - sbase[0]);
-        parallel_for(ng, [&](int gi) {
-            const FGroup &g = cp->fg[gi];
-            int base = gbase[gi];
-            for (size_t k = 0; k < g.blk.size(); ++k) {
-                const FBlk &fb = g.blk[k];
-                Strip &st = comb->strips[sbase[gi] + k];
-                st.dst = fb.lf;
-                st.rows = s.lsize(fb.lb);
-                st.cols = s.lsize(fb.lk);
-                st.ldd = fb.ld;
-                st.s0 = base;
-                st.s1 = base + cnt[gi][k];
-                base = st.s1;
-                comb_key[sbase[gi] - sbase[0] + k] = ((uint64_t)fb.lb << 32) | (uint32_t)fb.lk;
-            }
-        });
         comb->srcs.resize(gbase[ng]);
-        // 5. (parallel) sources of each block, in member order, into the group's range
-        parallel_for(ng, [&](int gi) {
-            const FGroup &g = cp->fg[gi];
-            const size_t nb = g.blk.size();
-            thread_local std::vector<int> slot, pos;
-            slot.assign((size_t)nl * nl, -1);
-            pos.assign(nb, 0);
-            int base = gbase[gi];
-            for (size_t k = 0; k < nb; ++k) {
-                slot[(size_t)g.blk[k].lk * nl + g.blk[k].lb] = (int)k;
-                pos[k] = base;
-                base += cnt[gi][k];
-            }
-            for (auto &m : g.mem)
-                for (auto &a : blk[m.first]) {
-                    int k = slot[(size_t)a.lk * nl + a.lb];
-                    if (k >= 0) comb->srcs[pos[k]++] = {t.la_off[a.lk] + a.row, t.Mtot[a.lk], m.second};
+        std::vector<uint32_t> comb_key(sbase[ng] - s0);  // lk * nl + lb: strips reading one LA_lk row range run together
+        // 4. (parallel) each output's strips and, in member order, its sources
+        parallel_for(
+            ng,
+            [&](int gi) {
+                const FOut &o = cp->fo[gi];
+                thread_local std::vector<int> pos;  // [lb][in][lk]
+                const size_t ni = o.in.size();
+                pos.assign(ni * nl * nl, -1);
+                int base = gbase[gi];
+                size_t st_i = sbase[gi];
+                for (auto &r : o.rows) {
+                    const Panel &pn = panels[r.panel];
+                    int k = 0;
+                    for (auto &c : r.chunk) {
+                        Strip &st = comb->strips[st_i];
+                        st.dst = pn.lf + r.row + (int64_t)k * pn.rows;
+                        st.rows = s.lsize(r.lb);
+                        st.cols = s.lsize(c.lk);
+                        st.ldd = pn.rows;
+                        st.s0 = base;
+                        st.s1 = base + c.nsrc;
+                        pos[((size_t)r.lb * ni + c.in) * nl + c.lk] = base;
+                        base = st.s1;
+                        k += s.lsize(c.lk);
+                        comb_key[st_i++ - s0] = (uint32_t)(c.lk * nl + r.lb);
+                    }
                 }
-        });
-    }
-    if (comb) {
-        if (comb_key.size() != comb->strips.size()) throw std::runtime_error("combination strip list out of step");
+                for_sources(o, [&](int q, const A &a, double c) {
+                    comb->srcs[pos[((size_t)a.lb * ni + q) * nl + a.lk]++] = {t.la_off[a.lk] + a.row, t.Mtot[a.lk], c};
+                });
+            },
+            4, 1);
         // stable counting sort by (lk, lb)
-        std::vector<int> start((size_t)nl * nl + 1, 0);
-        for (uint64_t k : comb_key) ++start[(size_t)(uint32_t)k * nl + (k >> 32) + 1];
+        std::vector<size_t> start((size_t)nl * nl + 1, 0);
+        for (uint32_t k : comb_key) ++start[k + 1];
         for (size_t b = 1; b < start.size(); ++b) start[b] += start[b - 1];
         TaskVec<Strip> sorted(comb->strips.size());
-        for (size_t i = 0; i < comb_key.size(); ++i)
-            sorted[start[(size_t)(uint32_t)comb_key[i] * nl + (comb_key[i] >> 32)]++] = comb->strips[i];
+        std::copy_n(comb->strips.begin(), s0, sorted.begin());
+        for (size_t i = 0; i < comb_key.size(); ++i) sorted[s0 + start[comb_key[i]]++] = comb->strips[s0 + i];
         comb->strips.swap(sorted);
     }
     // row maps of the fused panels: each panel's rows at a known offset, filled in parallel
@@ -818,18 +895,18 @@ TLay t_layout(const Site &s, const BLayout &L, const PRP &prp, ColProg *cp, std:
     }
     for (size_t k = 0; k < panels.size(); ++k) {
         const Panel &pn = panels[k];
-        int rsz = s.rsize(pn.ar), ksz = s.lsize(pn.lk);
-        t.gemm_flops += 2.0 * pn.rows * rsz * ksz;
+        const int rsz = s.rsize(pn.ar);
+        t.gemm_flops += 2.0 * pn.rows * rsz * pn.K;
         if (!g1) continue;
         GemmGroup g{};
         g.a = pn.lf;
-        g.b = prp.off[pn.lk] + (int64_t)(s.pbr[(size_t)pn.pin * s.nr + pn.ar] + pn.row * rsz) * ksz;
+        g.b = pn.pb;
         g.c = pn.tf;
         g.M = pn.rows;
         g.N = rsz;
-        g.K = ksz;
+        g.K = pn.K;
         g.lda = pn.rows;
-        g.ldb = ksz;
+        g.ldb = pn.K;
         g.ldc = pn.rows;
         g.rowmap = map0[k] + 1;
         add_gemm(*g1, g, tm, tn, kc);
@@ -867,7 +944,7 @@ void for_column_blocks(const Site &s, const TLay &t, const std::vector<CTerm> &t
 }
 
 // lbtm W application for column b2 (apply_op.hpp:23-101; abelian apply_op.hpp:24-139):
-// raw sources of the direct terms and of the fused groups, sorted by strip.
+// raw sources of the direct terms and of the fused outputs, sorted by strip.
 void lbtm_column(const Site &s, const TLay &t, const ColProg *cp, const std::vector<CTerm> &terms, int b2,
                  std::vector<Raw> &raw) {
     raw.clear();
@@ -889,16 +966,10 @@ void lbtm_column(const Site &s, const TLay &t, const ColProg *cp, const std::vec
     });
     if (cp)
         for (int gi : cp->fcol[b2]) {
-            const FGroup &g = cp->fg[gi];
-            for (auto &fb : g.blk) {
-                int i = spin2(s.left.q[fb.lb]), j = spin2(s.left.q[fb.lk]);
-                int jp = spin2(s.right.q[fb.ar]), ip = spin2(s.right.q[fb.al]);
-                const std::array<double, 4> &cpl =
-                    s.su2 ? coupling(j, std::abs(j - jp), jp, g.a, g.k, ap, i, std::abs(i - ip), ip) : one;
-                double coef = s.su2 ? cpl[case_of(g.rspin, g.cspin)] : 1.0;
-                int row0 = s.pbl[(size_t)g.pout * s.nl + fb.lb] + g.col * s.lsize(fb.lb);
-                raw.push_back({fb.al, fb.ar, row0, fb.tf, s.lsize(fb.lb), coef});
-            }
+            const FOut &o = cp->fo[gi];
+            for (auto &r : o.rows)
+                raw.push_back({r.al, r.ar, s.pbl[(size_t)o.pout * s.nl + r.lb] + o.col * s.lsize(r.lb), r.tf,
+                               s.lsize(r.lb), 1.0});
         }
     std::sort(raw.begin(), raw.end(), [](const Raw &x, const Raw &y) {
         if (x.al != y.al) return x.al < y.al;
@@ -1118,21 +1189,29 @@ void order_tiles(GemmList &gl) {
 void make_packs(StripList &sl) {
     sl.packs.clear();
     const int n = (int)sl.strips.size();
+    auto elems = [&](int i) { return (int64_t)sl.strips[i].rows * sl.strips[i].cols; };
+    auto chain = [&](int i) { return elems(i) <= kPackElems && sl.strips[i].s1 - sl.strips[i].s0 >= kChainSrcs; };
     int i = 0;
     while (i < n) {
-        sl.packs.push_back(i);
-        int64_t el = (int64_t)sl.strips[i].rows * sl.strips[i].cols;
+        int64_t el = elems(i);
+        if (el >= INT32_MAX - kPassElems) throw std::runtime_error("strip too large");
         int j = i + 1;
-        if (el <= kPackElems)
-            while (j < n && j - i < kPackStrips) {
-                const int64_t e = (int64_t)sl.strips[j].rows * sl.strips[j].cols;
-                if (el + e > kPackElems) break;
-                el += e;
+        if (el > kPackElems) {
+            for (int e = 0; e < el; e += kPassElems) sl.packs.push_back({i, 1, e});
+        } else if (chain(i)) {
+            while (j < n && j - i < 4 && chain(j)) ++j;
+            sl.packs.push_back({i, j - i, kPackWaves});
+        } else {
+            while (j < n && j - i < kPackStrips && !chain(j)) {
+                if (el + elems(j) > kPackElems) break;
+                el += elems(j);
                 ++j;
             }
+            if (j - i == 1) sl.packs.push_back({i, 1, 0});
+            else sl.packs.push_back({i, j - i, kPackSmall});
+        }
         i = j;
     }
-    sl.packs.push_back(n);
 }
 
 // ---------------- several vectors per launch ------------------------------
@@ -1191,9 +1270,9 @@ HostPlan build_sigma_plan(const mq_site_desc &d, int tm, int tn, int kc, FuseRul
     P.symm = s.symm;
     P.vec_len = s.X.total;
     PRP prp = prp_layout(s, P.reshape);
-    P.n_prp = prp.total;
     ColProg cp = column_program(s, false, fuse);
-    TLay t = t_layout(s, L, prp, &cp, &P.arrL, &P.combL, &P.g1, tm, tn, kc);
+    TLay t = t_layout(s, L, prp, &cp, &P.arrL, &P.reshape, &P.combL, &P.g1, tm, tn, kc);
+    P.n_prp = prp.total;
     P.n_la = t.la_total;
     P.n_t = t.t_total;
     std::vector<int> K(s.nr, 0);
@@ -1203,7 +1282,7 @@ HostPlan build_sigma_plan(const mq_site_desc &d, int tm, int tn, int kc, FuseRul
     const bool ref_lbtm =
         ref_count && (s.symm != MQ_SYMM_SU2U1 || (s.W.rows - s.W.one_rows) < (s.W.cols - s.W.one_cols));
     TLay tall;
-    if (ref_lbtm) tall = t_layout(s, L, prp, nullptr, nullptr, nullptr, nullptr, tm, tn, kc);
+    if (ref_lbtm) tall = t_layout(s, L, prp, nullptr, nullptr, nullptr, nullptr, nullptr, tm, tn, kc);
     double ref_axpy = 0, ref_trim = 0;
     ref_axpy = column_strips(
         s, t, cp, false, [&](int b2) { return ref_lbtm ? reference_axpy_flops(s, tall, b2) : 0.0; },
@@ -1294,11 +1373,11 @@ HostPlan build_lstep_plan(const mq_site_desc &d, int tm, int tn, int kc, FuseRul
     P.symm = s.symm;
     P.vec_len = s.X.total;
     PRP prp = prp_layout(s, P.reshape);
-    P.n_prp = prp.total;
     ColProg cp = column_program(s, true, fuse);
-    TLay t = t_layout(s, L, prp, &cp, &P.arrL, &P.combL, &P.g1, tm, tn, kc);
+    TLay t = t_layout(s, L, prp, &cp, &P.arrL, &P.reshape, &P.combL, &P.g1, tm, tn, kc);
+    P.n_prp = prp.total;
     TLay tall;
-    if (ref_count) tall = t_layout(s, L, prp, nullptr, nullptr, nullptr, nullptr, tm, tn, kc);
+    if (ref_count) tall = t_layout(s, L, prp, nullptr, nullptr, nullptr, nullptr, nullptr, tm, tn, kc);
     P.n_la = t.la_total;
     P.n_t = t.t_total;
     double axf = 0;
@@ -1851,7 +1930,7 @@ double reference_sigma_flops(const mq_site_desc &d) {
     bool lbtm = s.symm != MQ_SYMM_SU2U1 || (s.W.rows - s.W.one_rows) < (s.W.cols - s.W.one_cols);
     double f = 0;
     if (lbtm) {
-        TLay t = t_layout(s, L, prp, nullptr, nullptr, nullptr, nullptr, 64, 64, 1 << 30);
+        TLay t = t_layout(s, L, prp, nullptr, nullptr, nullptr, nullptr, nullptr, 64, 64, 1 << 30);
         f += t.gemm_flops;
         std::vector<Raw> raw;
         for (int b2 = 0; b2 < s.W.cols; ++b2) {

@@ -119,14 +119,21 @@ struct GemmList {
         return (int)b;
     }
 };
-// Consecutive strips are run in packs of one workgroup each: a pack is either
-// one strip of more than kPackElems elements, or up to kPackStrips strips of
-// together at most kPackElems elements (the fragmented blocks of small sectors).
-constexpr int kPackStrips = 64, kPackElems = 1024;
+// Strips are run in packs of one workgroup each: up to kPackStrips consecutive strips of
+// together at most kPackElems elements (the fragmented blocks of small sectors), up to
+// four such strips with at least kChainSrcs sources each (one wave per strip: its source
+// records are then read once per wave instead of by every element), or kPassElems
+// elements of one strip, from e0 on.
+constexpr int kPackStrips = 64, kPackElems = 1024, kPassElems = 2048, kChainSrcs = 8;
+constexpr int kPackSmall = -1, kPackWaves = -2;
+struct Pack {
+    int first, n;  // strips [first, first + n)
+    int e0;        // kPackSmall, kPackWaves, or the first element of the one strip's pass
+};
 struct StripList {
     TaskVec<Strip> strips;
     TaskVec<Src> srcs;
-    std::vector<int> packs;  // pack p runs strips [packs[p], packs[p + 1])
+    std::vector<Pack> packs;
 };
 // (re)compute the packs of a strip list, keeping the strip order
 void make_packs(StripList &sl);
