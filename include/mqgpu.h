@@ -415,6 +415,7 @@ int mq_gemm_f32(mq_ctx *ctx, int transA, int transB, int M, int N, int K,
  * step, 2 right step, 3 diagonal, plus MQ_HOST_FUSE(v), MQ_HOST_FUSE_RATIO(r)
  * and MQ_HOST_FUSE_MIN(m) to build with those MQ_OPT_FUSE* values (0 keeps a
  * default), and MQ_HOST_SCHED_REFERENCE for the reference's per-site schedule.  Arrays stay owned by the handle. */
+#define MQ_HOST_GATHER 16 /* sigma plans in the form the device runs: the output GEMM gathers its operand */
 #define MQ_HOST_FUSE(v) (((v) + 1) << 8)
 #define MQ_HOST_FUSE_RATIO(r) ((r) << 10) /* 1..255 */
 #define MQ_HOST_FUSE_MIN(m) ((m) << 18)   /* 1..4095 */
@@ -425,7 +426,8 @@ enum mq_plan_part {
     MQ_PART_G1_TILES = 4, MQ_PART_STRIPS = 5, MQ_PART_SRCS = 6, MQ_PART_G2_GROUPS = 7,
     MQ_PART_G2_TILES = 8, MQ_PART_SCATTER = 9, MQ_PART_COMB_STRIPS = 10, MQ_PART_COMB_SRCS = 11,
     MQ_PART_G1_ROWMAP = 12, MQ_PART_G2_ROWMAP = 13,
-    MQ_PART_LIVE = 14 /* sigma plans: the mq_plan_live_mask bytes */
+    MQ_PART_LIVE = 14, /* sigma plans: the mq_plan_live_mask bytes */
+    MQ_PART_GATHER_SRCS = 15, MQ_PART_GATHER_QUADS = 16, MQ_PART_GATHER_ROWS = 17 /* with MQ_HOST_GATHER */
 };
 int mq_host_plan_create(const mq_site_desc *desc, int kind, mq_host_plan **out);
 int mq_host_plan_part(const mq_host_plan *hp, int part, const void **ptr, int64_t *count, int64_t *elem_bytes);

@@ -86,12 +86,17 @@ struct DevArray {
     ~DevArray() { free_(); }
 };
 
+void check(hipError_t e, const char *what) {
+    if (e != hipSuccess) throw std::runtime_error(std::string(what) + ": " + hipGetErrorString(e));
+}
+
 struct DevGemm {
     DevArray<GemmGroup> groups;
     DevArray<GemmTile> tiles;
     DevArray<int> split;
     DevArray<RowMap> rowmap;
     int ntiles = 0, nsplit = 0, rblocks = 0;
+    std::vector<int> sp;  // host list of the copy under way
     void upload(const GemmList &g, hipStream_t s) {
         for (auto &x : g.groups) {
             if ((x.tm != 64 && x.tm != 128) || x.tn < 16 || x.tn > 128 || x.tn % 16 != 0)
@@ -104,7 +109,6 @@ struct DevGemm {
             if (t.g >= (int)g.groups.size()) throw std::runtime_error("GEMM tile outside the group list");
         groups.upload(g.groups, s);
         tiles.upload(g.tiles, s);
-        std::vector<int> sp;
         for (size_t i = 0; i < g.groups.size(); ++i)
             if (g.groups[i].split > 1) sp.push_back((int)i);
         split.upload(sp, s);
@@ -112,11 +116,30 @@ struct DevGemm {
         nsplit = (int)sp.size();
         rblocks = g.reduce_blocks();
     }
+    // C = op(A) op(B) for every group, in one launch
+    void run(const double *A, const double *B, double *C, double *W, int stage, hipStream_t s, bool = false) const {
+        if (ntiles)
+            check(launch_gemm(groups.p, tiles.p, ntiles, split.p, nsplit, rblocks, A, B, C, W, rowmap.p, stage, s),
+                  "GEMM");
+    }
+    void run(const float *A, const float *B, float *C, float *W, int stage, hipStream_t s, bool x3) const {
+        if (ntiles)
+            check(launch_gemm(groups.p, tiles.p, ntiles, split.p, nsplit, rblocks, A, B, C, W, rowmap.p, stage, s, x3),
+                  "GEMM");
+    }
+    void run(const float *A, const float *B, double *C, float *W, int stage, hipStream_t s, bool x3) const {
+        if (ntiles)
+            check(launch_gemm(groups.p, tiles.p, ntiles, split.p, nsplit, rblocks, A, B, C, W, rowmap.p, stage, s, x3),
+                  "GEMM");
+    }
+    // the same with the A operand gathered (HostPlan::gather)
+    template <class T>
+    void run_gather(const GatherSrc *src, const GatherQuad *quad, const GatherRow *row, const T *A, const T *B,
+                    double *C, T *W, hipStream_t s, bool x3) const {
+        check(launch_gemm_gather(groups.p, tiles.p, ntiles, split.p, nsplit, rblocks, A, B, C, W, src, quad, row, s, x3),
+              "gathered GEMM");
+    }
 };
-
-void check(hipError_t e, const char *what) {
-    if (e != hipSuccess) throw std::runtime_error(std::string(what) + ": " + hipGetErrorString(e));
-}
 
 // packs must cover the strips and their elements in order
 void check_packs(const StripList &sl) {
@@ -153,6 +176,9 @@ struct mq_plan {
     DevArray<Src> srcs, csrcs;
     DevArray<Pack> packs, cpacks;  // strip packs of wapply / combL
     DevGemm g1, g2;
+    DevArray<GatherSrc> gsrc;  // gathered A operand of g2 (HostPlan::gather)
+    DevArray<GatherQuad> gquad;
+    DevArray<GatherRow> grow;
     DevArray<double> la, rb, prp, t, c, tmp, ws;
     double w_src_el = 0, w_dst_el = 0;  // W-application source / destination elements
     const double *bound_L = nullptr, *bound_R = nullptr;
@@ -289,7 +315,7 @@ static int make_plan(mq_ctx *ctx, const mq_site_desc *desc, mq_plan **out, int k
         p->ctx = ctx;
         const int tm = ctx->tile_m, tn = ctx->tile_n, kc = ctx->kchunk;
         if (kind == PLAN_SIGMA)
-            p->hp = build_sigma_plan(*desc, tm, tn, kc, ctx->fuse, ctx->ref_flops != 0, ctx->schedule);
+            p->hp = build_sigma_plan(*desc, tm, tn, kc, ctx->fuse, ctx->ref_flops != 0, ctx->schedule, true);
         else if (kind == PLAN_LSTEP) p->hp = build_lstep_plan(*desc, tm, tn, kc, ctx->fuse, ctx->ref_flops != 0);
         else if (kind == PLAN_RSTEP) p->hp = build_rstep_plan(*desc, tm, tn, kc);
         else p->hp = build_diag_plan(*desc, tm, tn, kc);
@@ -311,6 +337,13 @@ static int make_plan(mq_ctx *ctx, const mq_site_desc *desc, mq_plan **out, int k
         p->g2.upload(h.g2, s);
         p->la.alloc(h.n_la);
         p->rb.alloc(h.n_rb);
+        if (h.gathered) {
+            p->gsrc.upload(h.gather.src, s);
+            p->gquad.upload(h.gather.quad, s);
+            p->grow.upload(h.gather.row, s);
+            // RB's rows beyond a segment's width stay zero for the plan's life
+            if (h.n_rb) check(hipMemsetAsync(p->rb.p, 0, sizeof(double) * h.n_rb, s), "clear RB");
+        }
         p->prp.alloc(h.n_prp);
         // sigma plans allocate the FP64 T and C arenas with their first FP64 sigma
         // (the mixed forms use FP32 ones), so a plan run only in a mixed form never
@@ -464,30 +497,22 @@ static void sigma_stages(mq_plan *p, const double *x, double *y, int prec, hipEv
         if (prec == MQ_PREC_FP64) {
             check(launch_copy2d(p->reshape.p, (int)h.reshape.size(), x, p->prp.p, s, true), "copy psi");
             mark(2);
-            check(launch_gemm(p->g1.groups.p, p->g1.tiles.p, p->g1.ntiles, p->g1.split.p, p->g1.nsplit, p->g1.rblocks, p->prp.p,
-                              p->rb.p, p->t.p, p->ws.p, p->g1.rowmap.p, ST_SIGMA, s),
-                  "gemm t");
+            p->g1.run(p->prp.p, p->rb.p, p->t.p, p->ws.p, ST_SIGMA, s);
             mark(3);
             check(launch_wapply(p->strips.p, p->packs.p, npacks(h.wapply), p->srcs.p, p->t.p, p->c.p, ST_SIGMA, s),
                   "W apply");
             mark(4);
-            check(launch_gemm(p->g2.groups.p, p->g2.tiles.p, p->g2.ntiles, p->g2.split.p, p->g2.nsplit, p->g2.rblocks, p->la.p,
-                              p->c.p, p->tmp.p, p->ws.p, p->g2.rowmap.p, ST_SIGMA_OUT, s),
-                  "gemm L");
+            p->g2.run(p->la.p, p->c.p, p->tmp.p, p->ws.p, ST_SIGMA_OUT, s);
         } else {
             check(launch_copy2d(p->reshape.p, (int)h.reshape.size(), x, p->prp32.p, s, true), "copy psi");
             mark(2);
-            check(launch_gemm(p->g1.groups.p, p->g1.tiles.p, p->g1.ntiles, p->g1.split.p, p->g1.nsplit, p->g1.rblocks, p->prp32.p,
-                              p->rb32.p, p->t32.p, p->ws32.p, p->g1.rowmap.p, ST_SIGMA, s, x3),
-                  "gemm t");
+            p->g1.run(p->prp32.p, p->rb32.p, p->t32.p, p->ws32.p, ST_SIGMA, s, x3);
             mark(3);
             check(launch_wapply(p->strips.p, p->packs.p, npacks(h.wapply), p->srcs.p, p->t32.p, p->c32.p, ST_SIGMA,
                                 s),
                   "W apply");
             mark(4);
-            check(launch_gemm(p->g2.groups.p, p->g2.tiles.p, p->g2.ntiles, p->g2.split.p, p->g2.nsplit, p->g2.rblocks, p->la32.p,
-                              p->c32.p, p->tmp.p, p->ws32.p, p->g2.rowmap.p, ST_SIGMA_OUT, s, x3),
-                  "gemm L");
+            p->g2.run(p->la32.p, p->c32.p, p->tmp.p, p->ws32.p, ST_SIGMA_OUT, s, x3);
         }
         check(launch_copy2d(p->scatter.p, (int)h.scatter.size(), p->tmp.p, y, s, true), "reshape sigma");
         mark(5);
@@ -496,29 +521,21 @@ static void sigma_stages(mq_plan *p, const double *x, double *y, int prec, hipEv
     if (prec == MQ_PREC_FP64) {
         check(launch_copy2d(p->reshape.p, (int)h.reshape.size(), x, p->prp.p, s, true), "reshape");
         mark(2);
-        check(launch_gemm(p->g1.groups.p, p->g1.tiles.p, p->g1.ntiles, p->g1.split.p, p->g1.nsplit, p->g1.rblocks, p->la.p,
-                          p->prp.p, p->t.p, p->ws.p, p->g1.rowmap.p, ST_SIGMA, s),
-              "gemm T");
+        p->g1.run(p->la.p, p->prp.p, p->t.p, p->ws.p, ST_SIGMA, s);
         mark(3);
-        check(launch_wapply(p->strips.p, p->packs.p, npacks(h.wapply), p->srcs.p, p->t.p, p->c.p, ST_SIGMA, s),
+        check(launch_wapply(p->strips.p, p->packs.p, npacks(h.wapply), p->srcs.p, p->t.p, p->t.p, ST_SIGMA, s),
               "W apply");
         mark(4);
-        check(launch_gemm(p->g2.groups.p, p->g2.tiles.p, p->g2.ntiles, p->g2.split.p, p->g2.nsplit, p->g2.rblocks, p->c.p,
-                          p->rb.p, y, p->ws.p, p->g2.rowmap.p, ST_SIGMA_OUT, s),
-              "gemm R");
+        p->g2.run_gather(p->gsrc.p, p->gquad.p, p->grow.p, p->t.p, p->rb.p, y, p->ws.p, s, false);
     } else {
         check(launch_copy2d(p->reshape.p, (int)h.reshape.size(), x, p->prp32.p, s, true), "reshape");
         mark(2);
-        check(launch_gemm(p->g1.groups.p, p->g1.tiles.p, p->g1.ntiles, p->g1.split.p, p->g1.nsplit, p->g1.rblocks, p->la32.p,
-                          p->prp32.p, p->t32.p, p->ws32.p, p->g1.rowmap.p, ST_SIGMA, s, x3),
-              "gemm T");
+        p->g1.run(p->la32.p, p->prp32.p, p->t32.p, p->ws32.p, ST_SIGMA, s, x3);
         mark(3);
-        check(launch_wapply(p->strips.p, p->packs.p, npacks(h.wapply), p->srcs.p, p->t32.p, p->c32.p, ST_SIGMA, s),
+        check(launch_wapply(p->strips.p, p->packs.p, npacks(h.wapply), p->srcs.p, p->t32.p, p->t32.p, ST_SIGMA, s),
               "W apply");
         mark(4);
-        check(launch_gemm(p->g2.groups.p, p->g2.tiles.p, p->g2.ntiles, p->g2.split.p, p->g2.nsplit, p->g2.rblocks, p->c32.p,
-                          p->rb32.p, y, p->ws32.p, p->g2.rowmap.p, ST_SIGMA_OUT, s, x3),
-              "gemm R");
+        p->g2.run_gather(p->gsrc.p, p->gquad.p, p->grow.p, p->t32.p, p->rb32.p, y, p->ws32.p, s, x3);
     }
     mark(5);
 }
@@ -543,7 +560,7 @@ static mq_plan::BatchLists &batch_setup(mq_plan *p, int nvec, bool f32) {
         B->ncopies = (int64_t)h.reshape.size() * nvec;
         // per-vector operands advance by their arena size; shared ones (panels) by 0
         GemmList g1 = h.rbtm ? batch_gemm(h.g1, nvec, h.n_prp, 0, h.n_t) : batch_gemm(h.g1, nvec, 0, h.n_prp, h.n_t);
-        GemmList g2 = h.rbtm ? batch_gemm(h.g2, nvec, 0, h.n_c, h.n_tmp) : batch_gemm(h.g2, nvec, h.n_c, 0, h.vec_len);
+        GemmList g2 = h.rbtm ? batch_gemm(h.g2, nvec, 0, h.n_c, h.n_tmp) : batch_gemm(h.g2, nvec, h.n_t, 0, h.vec_len);
         if (h.rbtm) {
             B->scatter.upload(batch_copies(h.scatter, nvec, h.n_tmp, h.vec_len), s);
             B->nscatter = (int64_t)h.scatter.size() * nvec;
@@ -628,52 +645,36 @@ static void sigma_batch_launch(mq_plan *p, const double *L, const double *R, con
         const bool x3 = prec == MQ_PREC_BF16X3;
         if (prec == MQ_PREC_FP64) {
             check(launch_copy2d(B.reshape.p, (int)B.ncopies, X, B.prp.p, s, true), "copy psi");
-            check(launch_gemm(B.g1.groups.p, B.g1.tiles.p, B.g1.ntiles, B.g1.split.p, B.g1.nsplit, B.g1.rblocks, B.prp.p, p->rb.p,
-                              B.t.p, B.ws.p, B.g1.rowmap.p, ST_SIGMA, s),
-                  "gemm t");
+            B.g1.run(B.prp.p, p->rb.p, B.t.p, B.ws.p, ST_SIGMA, s);
             check(launch_wapply(p->strips.p, p->packs.p, npacks(h.wapply), p->srcs.p, B.t.p, B.c.p, ST_SIGMA, s, nvec,
                                 h.n_t, h.n_c),
                   "W apply");
-            check(launch_gemm(B.g2.groups.p, B.g2.tiles.p, B.g2.ntiles, B.g2.split.p, B.g2.nsplit, B.g2.rblocks, p->la.p, B.c.p,
-                              A.tmp.p, B.ws.p, B.g2.rowmap.p, ST_SIGMA_OUT, s),
-                  "gemm L");
+            B.g2.run(p->la.p, B.c.p, A.tmp.p, B.ws.p, ST_SIGMA_OUT, s);
         } else {
             check(launch_copy2d(B.reshape.p, (int)B.ncopies, X, B.prp32.p, s, true), "copy psi");
-            check(launch_gemm(B.g1.groups.p, B.g1.tiles.p, B.g1.ntiles, B.g1.split.p, B.g1.nsplit, B.g1.rblocks, B.prp32.p,
-                              p->rb32.p, B.t32.p, B.ws32.p, B.g1.rowmap.p, ST_SIGMA, s, x3),
-                  "gemm t");
+            B.g1.run(B.prp32.p, p->rb32.p, B.t32.p, B.ws32.p, ST_SIGMA, s, x3);
             check(launch_wapply(p->strips.p, p->packs.p, npacks(h.wapply), p->srcs.p, B.t32.p, B.c32.p, ST_SIGMA, s,
                                 nvec, h.n_t, h.n_c),
                   "W apply");
-            check(launch_gemm(B.g2.groups.p, B.g2.tiles.p, B.g2.ntiles, B.g2.split.p, B.g2.nsplit, B.g2.rblocks, p->la32.p,
-                              B.c32.p, A.tmp.p, B.ws32.p, B.g2.rowmap.p, ST_SIGMA_OUT, s, x3),
-                  "gemm L");
+            B.g2.run(p->la32.p, B.c32.p, A.tmp.p, B.ws32.p, ST_SIGMA_OUT, s, x3);
         }
         check(launch_copy2d(Bl.scatter.p, (int)Bl.nscatter, A.tmp.p, Y, s, true), "reshape sigma");
         return;
     }
     if (prec == MQ_PREC_FP64) {
         check(launch_copy2d(B.reshape.p, (int)B.ncopies, X, B.prp.p, s, true), "reshape");
-        check(launch_gemm(B.g1.groups.p, B.g1.tiles.p, B.g1.ntiles, B.g1.split.p, B.g1.nsplit, B.g1.rblocks, p->la.p, B.prp.p,
-                          B.t.p, B.ws.p, B.g1.rowmap.p, ST_SIGMA, s),
-              "gemm T");
-        check(launch_wapply(p->strips.p, p->packs.p, npacks(h.wapply), p->srcs.p, B.t.p, B.c.p, ST_SIGMA, s, nvec,
-                            h.n_t, h.n_c),
+        B.g1.run(p->la.p, B.prp.p, B.t.p, B.ws.p, ST_SIGMA, s);
+        check(launch_wapply(p->strips.p, p->packs.p, npacks(h.wapply), p->srcs.p, B.t.p, B.t.p, ST_SIGMA, s, nvec,
+                            h.n_t, h.n_t),
               "W apply");
-        check(launch_gemm(B.g2.groups.p, B.g2.tiles.p, B.g2.ntiles, B.g2.split.p, B.g2.nsplit, B.g2.rblocks, B.c.p, p->rb.p, Y,
-                          B.ws.p, B.g2.rowmap.p, ST_SIGMA_OUT, s),
-              "gemm R");
+        B.g2.run_gather(p->gsrc.p, p->gquad.p, p->grow.p, B.t.p, p->rb.p, Y, B.ws.p, s, false);
     } else {
         check(launch_copy2d(B.reshape.p, (int)B.ncopies, X, B.prp32.p, s, true), "reshape");
-        check(launch_gemm(B.g1.groups.p, B.g1.tiles.p, B.g1.ntiles, B.g1.split.p, B.g1.nsplit, B.g1.rblocks, p->la32.p,
-                          B.prp32.p, B.t32.p, B.ws32.p, B.g1.rowmap.p, ST_SIGMA, s, prec == MQ_PREC_BF16X3),
-              "gemm T");
-        check(launch_wapply(p->strips.p, p->packs.p, npacks(h.wapply), p->srcs.p, B.t32.p, B.c32.p, ST_SIGMA, s,
-                            nvec, h.n_t, h.n_c),
+        B.g1.run(p->la32.p, B.prp32.p, B.t32.p, B.ws32.p, ST_SIGMA, s, prec == MQ_PREC_BF16X3);
+        check(launch_wapply(p->strips.p, p->packs.p, npacks(h.wapply), p->srcs.p, B.t32.p, B.t32.p, ST_SIGMA, s,
+                            nvec, h.n_t, h.n_t),
               "W apply");
-        check(launch_gemm(B.g2.groups.p, B.g2.tiles.p, B.g2.ntiles, B.g2.split.p, B.g2.nsplit, B.g2.rblocks, B.c32.p,
-                          p->rb32.p, Y, B.ws32.p, B.g2.rowmap.p, ST_SIGMA_OUT, s, prec == MQ_PREC_BF16X3),
-              "gemm R");
+        B.g2.run_gather(p->gsrc.p, p->gquad.p, p->grow.p, B.t32.p, p->rb32.p, Y, B.ws32.p, s, prec == MQ_PREC_BF16X3);
     }
 }
 
@@ -827,8 +828,8 @@ int mq_sigma_timed(mq_plan *plan, const double *L, const double *R, const double
                 work[3] = es * (h.n_prp + h.n_rb + h.n_t);
                 work[5] = es * (h.n_c + h.n_la) + 8.0 * (2.0 * h.n_tmp + h.vec_len);
             } else {
-                work[3] = es * (h.n_la + h.n_prp + h.n_t);
-                work[5] = es * (h.n_c + h.n_rb) + 8.0 * h.vec_len;
+                work[3] = es * (h.n_la + h.n_prp + h.n_t - dstel);  // the T arena ends with the C strips
+                work[5] = es * (h.gather.elements + h.n_rb) + 8.0 * h.vec_len;
             }
         }
         return MQ_OK;
@@ -859,9 +860,7 @@ int mq_gemm_f64(mq_ctx *ctx, int transA, int transB, int M, int N, int K, const 
         dg.upload(gl, ctx->stream);
         DevArray<double> ws;
         ws.alloc((size_t)gl.ws);
-        check(launch_gemm(dg.groups.p, dg.tiles.p, dg.ntiles, dg.split.p, dg.nsplit, dg.rblocks, A, B, C, ws.p, dg.rowmap.p, ST_MISC,
-                          ctx->stream),
-              "gemm");
+        dg.run(A, B, C, ws.p, ST_MISC, ctx->stream);
         check(hipStreamSynchronize(ctx->stream), "gemm sync");
         return MQ_OK;
     } catch (std::exception &e) {
@@ -958,9 +957,7 @@ int mq_gemm_f32(mq_ctx *ctx, int transA, int transB, int M, int N, int K, const 
         dg.upload(gl, ctx->stream);
         DevArray<float> ws;
         ws.alloc((size_t)gl.ws);
-        check(launch_gemm(dg.groups.p, dg.tiles.p, dg.ntiles, dg.split.p, dg.nsplit, dg.rblocks, A, B, C, ws.p, dg.rowmap.p, ST_MISC,
-                          ctx->stream, bf16x3 != 0),
-              "gemm");
+        dg.run(A, B, C, ws.p, ST_MISC, ctx->stream, bf16x3 != 0);
         check(hipStreamSynchronize(ctx->stream), "gemm sync");
         return MQ_OK;
     } catch (std::exception &e) {
@@ -1063,26 +1060,18 @@ int mq_boundary_step(mq_plan *plan, const double *in, const double *A, double *o
         check(launch_copy2d(plan->reshape.p, (int)h.reshape.size(), A, plan->prp.p, s), "reshape");
         if (h.kind == PLAN_LSTEP) {
             arrange_left(plan, in, s);
-            check(launch_gemm(plan->g1.groups.p, plan->g1.tiles.p, plan->g1.ntiles, plan->g1.split.p,
-                              plan->g1.nsplit, plan->g1.rblocks, plan->la.p, plan->prp.p, plan->t.p, plan->ws.p, plan->g1.rowmap.p, ST_STEP, s),
-                  "gemm T");
+            plan->g1.run(plan->la.p, plan->prp.p, plan->t.p, plan->ws.p, ST_STEP, s);
             check(launch_wapply(plan->strips.p, plan->packs.p, npacks(h.wapply), plan->srcs.p, plan->t.p, plan->c.p,
                                 ST_STEP, s),
                   "W apply");
-            check(launch_gemm(plan->g2.groups.p, plan->g2.tiles.p, plan->g2.ntiles, plan->g2.split.p,
-                              plan->g2.nsplit, plan->g2.rblocks, plan->c.p, A, plan->tmp.p, plan->ws.p, plan->g2.rowmap.p, ST_STEP_OUT, s),
-                  "gemm out");
+            plan->g2.run(plan->c.p, A, plan->tmp.p, plan->ws.p, ST_STEP_OUT, s);
         } else {
             check(launch_copy2d(plan->arrR.p, (int)h.arrR.size(), in, plan->rb.p, s), "arrange R");
-            check(launch_gemm(plan->g1.groups.p, plan->g1.tiles.p, plan->g1.ntiles, plan->g1.split.p,
-                              plan->g1.nsplit, plan->g1.rblocks, A, plan->rb.p, plan->t.p, plan->ws.p, plan->g1.rowmap.p, ST_STEP, s),
-                  "gemm t");
+            plan->g1.run(A, plan->rb.p, plan->t.p, plan->ws.p, ST_STEP, s);
             check(launch_wapply(plan->strips.p, plan->packs.p, npacks(h.wapply), plan->srcs.p, plan->t.p, plan->c.p,
                                 ST_STEP, s),
                   "W apply");
-            check(launch_gemm(plan->g2.groups.p, plan->g2.tiles.p, plan->g2.ntiles, plan->g2.split.p,
-                              plan->g2.nsplit, plan->g2.rblocks, plan->c.p, plan->prp.p, plan->tmp.p, plan->ws.p, plan->g2.rowmap.p, ST_STEP_OUT, s),
-                  "gemm out");
+            plan->g2.run(plan->c.p, plan->prp.p, plan->tmp.p, plan->ws.p, ST_STEP_OUT, s);
         }
         check(launch_copy2d(plan->scatter.p, (int)h.scatter.size(), plan->tmp.p, out, s), "scatter");
         return MQ_OK;
@@ -1105,9 +1094,7 @@ int mq_diagonal(mq_plan *plan, const double *L, const double *R, double *diag) {
         check(launch_wapply(plan->strips.p, plan->packs.p, npacks(h.wapply), plan->srcs.p, plan->la.p, plan->t.p,
                             ST_MISC, s),
               "diagonal W apply");
-        check(launch_gemm(plan->g2.groups.p, plan->g2.tiles.p, plan->g2.ntiles, plan->g2.split.p, plan->g2.nsplit, plan->g2.rblocks,
-                          plan->t.p, plan->rb.p, diag, plan->ws.p, plan->g2.rowmap.p, ST_MISC, s),
-              "diagonal gemm");
+        plan->g2.run(plan->t.p, plan->rb.p, diag, plan->ws.p, ST_MISC, s);
         return MQ_OK;
     } catch (std::exception &e) {
         return fail(plan->ctx, e, MQ_ERR_HIP);
@@ -2105,13 +2092,13 @@ int mq_host_plan_create(const mq_site_desc *desc, int kind, mq_host_plan **out) 
     try {
         std::unique_ptr<mq_host_plan> h(new mq_host_plan());
         const int tm = 0, tn = 0, kc = 2048;
-        const int fm = (kind >> 8) & 3, fr = (kind >> 10) & 255, fmin = (kind >> 18) & 4095, k = kind & 255;
+        const int fm = (kind >> 8) & 3, fr = (kind >> 10) & 255, fmin = (kind >> 18) & 4095, k = kind & 15;
         FuseRule fuse;
         if (fm) fuse.mode = fm - 1;
         if (fr) fuse.ratio = fr;
         if (fmin) fuse.min_entries = fmin;
         const int sched = (kind >> 30) & 1;
-        if (k == PLAN_SIGMA) h->hp = build_sigma_plan(*desc, tm, tn, kc, fuse, true, sched);
+        if (k == PLAN_SIGMA) h->hp = build_sigma_plan(*desc, tm, tn, kc, fuse, true, sched, (kind & MQ_HOST_GATHER) != 0);
         else if (k == PLAN_LSTEP) h->hp = build_lstep_plan(*desc, tm, tn, kc, fuse);
         else if (k == PLAN_RSTEP) h->hp = build_rstep_plan(*desc, tm, tn, kc);
         else if (k == PLAN_DIAG) h->hp = build_diag_plan(*desc, tm, tn, kc);
@@ -2142,6 +2129,9 @@ int mq_host_plan_part(const mq_host_plan *h, int part, const void **ptr, int64_t
         case MQ_PART_COMB_SRCS: *ptr = p.combL.srcs.data(); *count = p.combL.srcs.size(); *elem = sizeof(Src); break;
         case MQ_PART_G1_ROWMAP: *ptr = p.g1.rowmap.data(); *count = p.g1.rowmap.size(); *elem = sizeof(RowMap); break;
         case MQ_PART_G2_ROWMAP: *ptr = p.g2.rowmap.data(); *count = p.g2.rowmap.size(); *elem = sizeof(RowMap); break;
+        case MQ_PART_GATHER_SRCS: *ptr = p.gather.src.data(); *count = p.gather.src.size(); *elem = sizeof(GatherSrc); break;
+        case MQ_PART_GATHER_QUADS: *ptr = p.gather.quad.data(); *count = p.gather.quad.size(); *elem = sizeof(GatherQuad); break;
+        case MQ_PART_GATHER_ROWS: *ptr = p.gather.row.data(); *count = p.gather.row.size(); *elem = sizeof(GatherRow); break;
         case MQ_PART_LIVE: *ptr = p.live.data(); *count = p.live.size(); *elem = 1; break;
         default: return MQ_ERR_ARG;
     }

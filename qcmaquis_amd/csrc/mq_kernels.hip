@@ -280,9 +280,16 @@ __device__ __forceinline__ void a_slot(int r, int &i, int &k) {
         k = ((int)threadIdx.x + 256 * r) / TM;
 }
 
+// The plain operands' loads are unconditional, at addresses clamped into the operands:
+// rows and columns past the edge give results that are not stored, and k past the end is
+// zeroed before the stash (gemm_mask).  A load under a condition sits in a block of its
+// own; without them the T GEMM of the L=24 m=512 centre takes 745 against 786 us (BF16x3)
+// and 768 against 797 (TwoU1, FP32), and FP64 the same 1,860.  The gathered form keeps
+// conditional loads (GATHER): there the columns past N and the empty row blocks are bytes
+// not read (FP64 1,291 against 1,392 us, BF16x3 561 against 611).
 template <int TM, int TN, class T, bool QUADS = false>
-__device__ __forceinline__ void gemm_fetch(const GemmGroup &g, const T *__restrict__ A, const T *__restrict__ B,
-                                           int m0, int n0, int k0, int kend, GemmStage<TM, TN, T> &st) {
+__device__ __forceinline__ void gemm_fetch_a(const GemmGroup &g, const T *__restrict__ A, int m0, int k0, int kend,
+                                             GemmStage<TM, TN, T> &st) {
     constexpr int TK = kstep<T>();
 #pragma unroll
     for (int r = 0; r < TM * TK / 256; ++r) {
@@ -294,11 +301,14 @@ __device__ __forceinline__ void gemm_fetch(const GemmGroup &g, const T *__restri
             k = e % TK;
             i = e / TK;
         }
-        const int gm = m0 + i, gk = k0 + k;
-        T v = 0;
-        if (gm < g.M && gk < kend) v = g.transA ? A[g.a + gk + (int64_t)gm * g.lda] : A[g.a + gm + (int64_t)gk * g.lda];
-        st.a[r] = v;
+        const int gm = min(m0 + i, g.M - 1), gk = min(k0 + k, kend - 1);
+        st.a[r] = g.transA ? A[g.a + gk + (int64_t)gm * g.lda] : A[g.a + gm + (int64_t)gk * g.lda];
     }
+}
+template <int TM, int TN, class T, bool GATHER>
+__device__ __forceinline__ void gemm_fetch_b(const GemmGroup &g, const T *__restrict__ B, int n0, int k0, int kend,
+                                             GemmStage<TM, TN, T> &st) {
+    constexpr int TK = kstep<T>();
 #pragma unroll
     for (int r = 0; r < TN * TK / 256; ++r) {
         const int e = threadIdx.x + 256 * r;
@@ -310,24 +320,127 @@ __device__ __forceinline__ void gemm_fetch(const GemmGroup &g, const T *__restri
             j = e % TN;
             k = e / TN;
         }
-        const int gn = n0 + j, gk = k0 + k;
-        T v = 0;
-        if (gn < g.N && gk < kend) v = g.transB ? B[g.b + gn + (int64_t)gk * g.ldb] : B[g.b + gk + (int64_t)gn * g.ldb];
-        st.b[r] = v;
+        if constexpr (GATHER) {
+            const int gn = n0 + j, gk = k0 + k;
+            T v = 0;
+            if (gn < g.N && gk < kend) v = B[g.b + gk + (int64_t)gn * g.ldb];
+            st.b[r] = v;
+        } else {
+            const int gn = min(n0 + j, g.N - 1), gk = min(k0 + k, kend - 1);
+            st.b[r] = g.transB ? B[g.b + gn + (int64_t)gk * g.ldb] : B[g.b + gk + (int64_t)gn * g.ldb];
+        }
+    }
+}
+// zeros for the k of a last step that lie past the end (kn of its k are inside)
+template <int TM, int TN, class T, bool QUADS>
+__device__ __forceinline__ void gemm_mask(const GemmGroup &g, int kn, GemmStage<TM, TN, T> &st) {
+    constexpr int TK = kstep<T>();
+    if (kn >= TK) return;
+#pragma unroll
+    for (int r = 0; r < TM * TK / 256; ++r) {
+        int i, k;
+        if (!g.transA) a_slot<TM, QUADS>(r, i, k);
+        else k = ((int)threadIdx.x + 256 * r) % TK;
+        st.a[r] = k < kn ? st.a[r] : (T)0;
+    }
+#pragma unroll
+    for (int r = 0; r < TN * TK / 256; ++r) {
+        const int e = threadIdx.x + 256 * r, k = !g.transB ? e % TK : e / TN;
+        st.b[r] = k < kn ? st.b[r] : (T)0;
     }
 }
 
-template <int TM, int TN, class T>
+// The gathered A operand (Gather, QUADS slots): a thread keeps one row of the tile and
+// takes whole quads of it, so a K step costs it TM / 64 source records.  Each link of the
+// chain quad -> source record -> elements is read one K step before the next one needs
+// it, so that no load waits for the one before it.
+struct GatherArgs {
+    const GatherSrc *src;
+    const GatherQuad *quad;
+    const GatherRow *row;
+};
+template <int TM, class T>
+struct GatherState {
+    static constexpr int NQ = TM / 64;
+    GatherRow row;
+    GatherQuad next[NQ];
+    GatherSrc src[NQ];
+    int k0[NQ], len[NQ];
+    T coef[NQ];
+    __device__ __forceinline__ void init(const GemmGroup &g, const GatherArgs ga, int m0) {
+        const int gm = m0 + (int)threadIdx.x % TM;
+        row = GatherRow{-1, 0, 0, 0};
+        if (gm < g.M) row = ga.row[g.grow + gm];
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+            src[q] = GatherSrc{-1, 0.0};
+            k0[q] = len[q] = 0;
+        }
+    }
+    // the quads of the K step at k: vector loads, though uniform over a wave (a scalar load
+    // in flight would make every LDS read of the products wait for it)
+    __device__ __forceinline__ void quads(const GemmGroup &g, const GatherArgs ga, int k, int kend) {
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+            const int kq = k + 4 * ((int)threadIdx.x / TM + (256 / TM) * q);
+            next[q] = GatherQuad{0, 0};
+            if (kq < kend) next[q] = ga.quad[g.gq + (kq >> 2)];
+        }
+    }
+    // One K step: the elements whose records were read last, the records of the step
+    // whose quads were read last, the quads of the step at k.  Every earlier load is
+    // consumed before the first new one is issued: the counter that a wave waits on is in
+    // order, so a wait in between would expose the new loads' whole latency.
+    template <int TN>
+    __device__ __forceinline__ void fetch(const GemmGroup &g, const T *__restrict__ A, const GatherArgs ga, int k,
+                                          int kend, GemmStage<TM, TN, T> &st) {
+        const T *a[NQ];
+        int n[NQ];
+        const GatherSrc *rec[NQ];
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+            coef[q] = (T)src[q].coef;
+            a[q] = A + g.a + src[q].off + row.row + (int64_t)k0[q] * row.ld;
+            n[q] = src[q].off >= 0 ? len[q] : 0;
+            k0[q] = next[q].k0len >> 3;
+            len[q] = row.strip >= 0 ? next[q].k0len & 7 : 0;
+            rec[q] = ga.src + next[q].desc + row.strip;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int q = 0; q < NQ; ++q)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) st.a[4 * q + u] = u < n[q] ? a[q][(int64_t)u * row.ld] : (T)0;
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+            src[q] = GatherSrc{-1, 0.0};
+            if (len[q] > 0) src[q] = *rec[q];
+        }
+        quads(g, ga, k, kend);
+    }
+    template <int TN>
+    __device__ __forceinline__ void scale(GemmStage<TM, TN, T> &st) const {
+#pragma unroll
+        for (int q = 0; q < NQ; ++q)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) st.a[4 * q + u] *= coef[q];
+    }
+};
+
+template <int TM, int TN, class T, bool QUADS = false>
 __device__ __forceinline__ void gemm_stash(const GemmGroup &g, const GemmStage<TM, TN, T> &st, T (*As)[TM + 2],
                                            T (*Bs)[TN + 2]) {
     constexpr int TK = kstep<T>();
 #pragma unroll
     for (int r = 0; r < TM * TK / 256; ++r) {
         const int e = threadIdx.x + 256 * r;
-        if (!g.transA)
-            As[e / TM][e % TM] = st.a[r];
-        else
+        if (!g.transA) {
+            int i, k;
+            a_slot<TM, QUADS>(r, i, k);
+            As[k][i] = st.a[r];
+        } else {
             As[e % TK][e / TK] = st.a[r];
+        }
     }
 #pragma unroll
     for (int r = 0; r < TN * TK / 256; ++r) {
@@ -431,13 +544,26 @@ __device__ __forceinline__ void store_rowmap_staged(const GemmGroup &g, int m0, 
     }
 }
 
+// The operands of the K step at k into registers.
+template <int TM, int TN, class T, bool X3, bool GATHER>
+__device__ __forceinline__ void gemm_next(const GemmGroup &g, const T *__restrict__ A, const T *__restrict__ B,
+                                          const GatherArgs ga, int m0, int n0, int k, int kend,
+                                          GemmStage<TM, TN, T> &st, GatherState<TM, T> &gs) {
+    if constexpr (GATHER)
+        gs.template fetch<TN>(g, A, ga, k + 2 * kstep<T>(), kend, st);
+    else
+        gemm_fetch_a<TM, TN, T, X3>(g, A, m0, k, kend, st);
+    gemm_fetch_b<TM, TN, T, GATHER>(g, B, n0, k, kend, st);
+}
+
 // T: operand type; TO: output type; partial tiles of split-K groups are
 // stored in T and summed by k_split_reduce.  X3 (T = float only): BF16x3 products.
-// STAGED: row-mapped groups store through LDS (store_rowmap_staged).
-template <int TM, int TN, class T, class TO, bool X3, bool STAGED>
+// STAGED: row-mapped groups store through LDS (store_rowmap_staged).  GATHER: A through
+// the gather lists.
+template <int TM, int TN, class T, class TO, bool X3, bool STAGED, bool GATHER>
 __device__ __forceinline__ void gemm_tile(const GemmGroup &g, const GemmTile &t, const T *__restrict__ A,
                                           const T *__restrict__ B, TO *__restrict__ C, T *__restrict__ W,
-                                          const RowMap *__restrict__ rowmap, double *lds) {
+                                          const RowMap *__restrict__ rowmap, const GatherArgs ga, double *lds) {
     static_assert(!X3 || sizeof(T) == 4, "BF16x3 products take FP32 operands");
     typedef Mfma<T> MF;
     constexpr int TK = kstep<T>();
@@ -460,18 +586,26 @@ __device__ __forceinline__ void gemm_tile(const GemmGroup &g, const GemmTile &t,
 #pragma unroll
         for (int j = 0; j < NJ; ++j) acc[i][j] = typename MF::acc{0, 0, 0, 0};
     GemmStage<TM, TN, T> st;
+    GatherState<TM, T> gs;
     int buf = 0;
     if (kbeg < kend) {
-        gemm_fetch<TM, TN, T, X3>(g, A, B, m0, n0, kbeg, kend, st);
+        if constexpr (GATHER) {
+            gs.init(g, ga, m0);
+            gs.quads(g, ga, kbeg, kend);
+            gs.template fetch<TN>(g, A, ga, kbeg + TK, kend, st);  // no records yet: reads none
+        }
+        gemm_next<TM, TN, T, X3, GATHER>(g, A, B, ga, m0, n0, kbeg, kend, st, gs);
+        if constexpr (GATHER) gs.template scale<TN>(st);
+        else gemm_mask<TM, TN, T, X3>(g, kend - kbeg, st);
         if constexpr (X3)
             gemm_stash_x3<TM, TN>(g, st, Ax[0], Bx[0]);
         else
-            gemm_stash<TM, TN, T>(g, st, As[0], Bs[0]);
+            gemm_stash<TM, TN, T, GATHER>(g, st, As[0], Bs[0]);
     }
     __syncthreads();
     for (int k0 = kbeg; k0 < kend; k0 += TK) {
         const bool more = k0 + TK < kend;
-        if (more) gemm_fetch<TM, TN, T, X3>(g, A, B, m0, n0, k0 + TK, kend, st);
+        if (more) gemm_next<TM, TN, T, X3, GATHER>(g, A, B, ga, m0, n0, k0 + TK, kend, st, gs);
         if constexpr (X3) {
             // one 16x16x16 step covers the K tile: lane group lq holds k = 4 lq .. 4 lq + 3
             Bf16Quad av[MI];
@@ -502,10 +636,12 @@ __device__ __forceinline__ void gemm_tile(const GemmGroup &g, const GemmTile &t,
             }
         }
         if (more) {
+            if constexpr (GATHER) gs.template scale<TN>(st);
+            else gemm_mask<TM, TN, T, X3>(g, kend - k0 - TK, st);
             if constexpr (X3)
                 gemm_stash_x3<TM, TN>(g, st, Ax[buf ^ 1], Bx[buf ^ 1]);
             else
-                gemm_stash<TM, TN, T>(g, st, As[buf ^ 1], Bs[buf ^ 1]);
+                gemm_stash<TM, TN, T, GATHER>(g, st, As[buf ^ 1], Bs[buf ^ 1]);
         }
         __syncthreads();
         buf ^= 1;
@@ -524,10 +660,12 @@ __device__ __forceinline__ void gemm_tile(const GemmGroup &g, const GemmTile &t,
             // row gm of C: column-major with ldc, or placed by the group's row map
             TO *out = C + g.c + gm;
             int64_t ld = g.ldc;
-            if (g.rowmap > 0) {
-                const RowMap rm = rowmap[g.rowmap - 1 + gm];
-                out = C + g.c + rm.off;
-                ld = rm.ld;
+            if constexpr (!GATHER) {
+                if (g.rowmap > 0) {
+                    const RowMap rm = rowmap[g.rowmap - 1 + gm];
+                    out = C + g.c + rm.off;
+                    ld = rm.ld;
+                }
             }
 #pragma unroll
             for (int j = 0; j < NJ; ++j)
@@ -556,19 +694,19 @@ __device__ __forceinline__ void gemm_tile(const GemmGroup &g, const GemmTile &t,
 }
 
 // Column tile widths are multiples of 16 up to 128.
-template <int TM, class T, class TO, bool X3, bool STAGED>
+template <int TM, class T, class TO, bool X3, bool STAGED, bool GATHER = false>
 __device__ __forceinline__ void gemm_tile_n(const GemmGroup &g, const GemmTile &t, const T *__restrict__ A,
                                             const T *__restrict__ B, TO *__restrict__ C, T *__restrict__ W,
-                                            const RowMap *__restrict__ rowmap, double *lds) {
+                                            const RowMap *__restrict__ rowmap, const GatherArgs ga, double *lds) {
     switch (g.tn) {
-        case 16: gemm_tile<TM, 16, T, TO, X3, STAGED>(g, t, A, B, C, W, rowmap, lds); break;
-        case 32: gemm_tile<TM, 32, T, TO, X3, STAGED>(g, t, A, B, C, W, rowmap, lds); break;
-        case 48: gemm_tile<TM, 48, T, TO, X3, STAGED>(g, t, A, B, C, W, rowmap, lds); break;
-        case 64: gemm_tile<TM, 64, T, TO, X3, STAGED>(g, t, A, B, C, W, rowmap, lds); break;
-        case 80: gemm_tile<TM, 80, T, TO, X3, STAGED>(g, t, A, B, C, W, rowmap, lds); break;
-        case 96: gemm_tile<TM, 96, T, TO, X3, STAGED>(g, t, A, B, C, W, rowmap, lds); break;
-        case 112: gemm_tile<TM, 112, T, TO, X3, STAGED>(g, t, A, B, C, W, rowmap, lds); break;
-        default: gemm_tile<TM, 128, T, TO, X3, STAGED>(g, t, A, B, C, W, rowmap, lds); break;
+        case 16: gemm_tile<TM, 16, T, TO, X3, STAGED, GATHER>(g, t, A, B, C, W, rowmap, ga, lds); break;
+        case 32: gemm_tile<TM, 32, T, TO, X3, STAGED, GATHER>(g, t, A, B, C, W, rowmap, ga, lds); break;
+        case 48: gemm_tile<TM, 48, T, TO, X3, STAGED, GATHER>(g, t, A, B, C, W, rowmap, ga, lds); break;
+        case 64: gemm_tile<TM, 64, T, TO, X3, STAGED, GATHER>(g, t, A, B, C, W, rowmap, ga, lds); break;
+        case 80: gemm_tile<TM, 80, T, TO, X3, STAGED, GATHER>(g, t, A, B, C, W, rowmap, ga, lds); break;
+        case 96: gemm_tile<TM, 96, T, TO, X3, STAGED, GATHER>(g, t, A, B, C, W, rowmap, ga, lds); break;
+        case 112: gemm_tile<TM, 112, T, TO, X3, STAGED, GATHER>(g, t, A, B, C, W, rowmap, ga, lds); break;
+        default: gemm_tile<TM, 128, T, TO, X3, STAGED, GATHER>(g, t, A, B, C, W, rowmap, ga, lds); break;
     }
 }
 
@@ -594,7 +732,7 @@ constexpr int gemm_kernel_lds_bytes() {
 // 122 VGPRs + 64 AGPRs (2 waves); within 170 registers it needs no spills, and the
 // third wave took the L=24 T GEMM from 1.33 to 1.16 ms (4 waves would spill).
 template <int STAGE, class T, class TO, bool X3>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(X3 ? 3 : 1))) k_gemm(const GemmGroup *__restrict__ groups, const GemmTile *__restrict__ tiles,
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(X3 ? 3 : sizeof(T) == 8 ? 2 : 1))) k_gemm(const GemmGroup *__restrict__ groups, const GemmTile *__restrict__ tiles,
                                               const T *__restrict__ A, const T *__restrict__ B, TO *__restrict__ C,
                                               T *__restrict__ W, const RowMap *__restrict__ rowmap) {
     constexpr bool staged = gemm_staged<STAGE, T, TO>();
@@ -603,9 +741,30 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(X3 ? 3
     if (t.g < 0) return;  // padding tile of the XCD-ordered list
     const GemmGroup g = groups[t.g];
     if (g.tm == 128)
-        gemm_tile_n<128, T, TO, X3, staged>(g, t, A, B, C, W, rowmap, lds);
+        gemm_tile_n<128, T, TO, X3, staged>(g, t, A, B, C, W, rowmap, GatherArgs{}, lds);
     else
-        gemm_tile_n<64, T, TO, X3, staged>(g, t, A, B, C, W, rowmap, lds);
+        gemm_tile_n<64, T, TO, X3, staged>(g, t, A, B, C, W, rowmap, GatherArgs{}, lds);
+}
+
+// The sigma's output GEMM with a gathered A operand: sigma_al = sum over K segments of
+// (T block or W-application strip) x RB.  Most C strips have a single source, one T block
+// times a coefficient (63 % of C at the L=24 m=512 centre, 85 % for TwoU1), and some
+// none; the W application wrote them to C and this GEMM read them back.  Gathering costs
+// the GEMM some time (source records, shorter runs: FP64 1,157 -> 1,291 us, BF16x3 500 ->
+// 561, TwoU1 FP32 640 -> 675) and takes the single-source strips out of the W
+// application (1,041 -> 338, 690 -> 198, 650 -> 27 us).
+template <class T, bool X3>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 3 : 2)))
+k_gemm_gather(const GemmGroup *__restrict__ groups, const GemmTile *__restrict__ tiles, const T *__restrict__ A,
+              const T *__restrict__ B, double *__restrict__ C, T *__restrict__ W, const GatherArgs ga) {
+    __shared__ double lds[(gemm_lds_bytes<T, X3>() + 7) / 8];
+    const GemmTile t = tiles[blockIdx.x];
+    if (t.g < 0) return;  // padding tile of the XCD-ordered list
+    const GemmGroup g = groups[t.g];
+    if (g.tm == 128)
+        gemm_tile_n<128, T, double, X3, false, true>(g, t, A, B, C, W, nullptr, ga, lds);
+    else
+        gemm_tile_n<64, T, double, X3, false, true>(g, t, A, B, C, W, nullptr, ga, lds);
 }
 
 // C = sum over splits of the partial tiles, in split order (deterministic),
@@ -917,6 +1076,35 @@ hipError_t launch_gemm(const GemmGroup *groups, const GemmTile *tiles, int ntile
                                                 s);
     return gemm_launch<float, double, false>(groups, tiles, ntiles, split_gids, nsplit, rblocks, A, B, C, W, rowmap, stage,
                                              s);
+}
+
+template <class T, bool X3>
+static hipError_t gather_launch(const GemmGroup *groups, const GemmTile *tiles, int ntiles, const int *split_gids,
+                                int nsplit, int rblocks, const T *A, const T *B, double *C, T *W,
+                                const GatherSrc *src, const GatherQuad *quad, const GatherRow *row, hipStream_t s) {
+    if (ntiles > 0)
+        hipLaunchKernelGGL((k_gemm_gather<T, X3>), dim3(ntiles), dim3(256), 0, s, groups, tiles, A, B, C, W,
+                           GatherArgs{src, quad, row});
+    if (nsplit > 0)
+        hipLaunchKernelGGL((k_split_reduce<ST_SIGMA_OUT, T, double>), dim3(rblocks, nsplit), dim3(256), 0, s, groups,
+                           split_gids, W, C);
+    return hipGetLastError();
+}
+hipError_t launch_gemm_gather(const GemmGroup *groups, const GemmTile *tiles, int ntiles, const int *split_gids,
+                              int nsplit, int rblocks, const double *A, const double *B, double *C, double *W,
+                              const GatherSrc *src, const GatherQuad *quad, const GatherRow *row, hipStream_t s,
+                              bool) {
+    return gather_launch<double, false>(groups, tiles, ntiles, split_gids, nsplit, rblocks, A, B, C, W, src, quad, row,
+                                        s);
+}
+hipError_t launch_gemm_gather(const GemmGroup *groups, const GemmTile *tiles, int ntiles, const int *split_gids,
+                              int nsplit, int rblocks, const float *A, const float *B, double *C, float *W,
+                              const GatherSrc *src, const GatherQuad *quad, const GatherRow *row, hipStream_t s,
+                              bool bf16x3) {
+    return bf16x3 ? gather_launch<float, true>(groups, tiles, ntiles, split_gids, nsplit, rblocks, A, B, C, W, src,
+                                               quad, row, s)
+                  : gather_launch<float, false>(groups, tiles, ntiles, split_gids, nsplit, rblocks, A, B, C, W, src,
+                                                quad, row, s);
 }
 
 hipError_t launch_multidot(const PairArgs &a, int npairs, int64_t n, int nblocks, double *partial, hipStream_t s) {

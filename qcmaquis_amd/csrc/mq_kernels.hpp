@@ -41,6 +41,15 @@ hipError_t launch_gemm(const GemmGroup *groups, const GemmTile *tiles, int ntile
 hipError_t launch_gemm(const GemmGroup *groups, const GemmTile *tiles, int ntiles, const int *split_gids, int nsplit, int rblocks,
                        const float *A, const float *B, double *C, float *W, const RowMap *rowmap, int stage,
                        hipStream_t s, bool bf16x3 = false);
+// the sigma's output GEMM of plans with a gathered A operand (HostPlan::gather)
+hipError_t launch_gemm_gather(const GemmGroup *groups, const GemmTile *tiles, int ntiles, const int *split_gids,
+                              int nsplit, int rblocks, const double *A, const double *B, double *C, double *W,
+                              const GatherSrc *src, const GatherQuad *quad, const GatherRow *row, hipStream_t s,
+                              bool bf16x3 = false);
+hipError_t launch_gemm_gather(const GemmGroup *groups, const GemmTile *tiles, int ntiles, const int *split_gids,
+                              int nsplit, int rblocks, const float *A, const float *B, double *C, float *W,
+                              const GatherSrc *src, const GatherQuad *quad, const GatherRow *row, hipStream_t s,
+                              bool bf16x3);
 // Davidson vector operations.  Vector pairs and coefficients are kernel arguments, at
 // most kCombMax per launch.
 constexpr int kCombMax = 48;

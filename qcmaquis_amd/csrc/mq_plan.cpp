@@ -1083,11 +1083,12 @@ int64_t walk_segment(const std::vector<std::pair<int, int>> &rs, const Raw *r0, 
 //  3. (parallel) the strips and sources are written at their places.
 // Strip dst offsets are relative to the al block start (patch_strips adds the C
 // arena offset of al once every K_al is known).  skip_rskip: the columns stored as
-// their hermitian partner are left out.  Returns the sum of extra over the columns.
+// their hermitian partner are left out.  kpad: every segment's K is rounded up to a
+// multiple of it.  Returns the sum of extra over the columns.
 template <class Extra, class Accept, class OnSeg>
 double column_strips(const Site &s, const TLay &t, const ColProg &cp, bool skip_rskip, Extra &&extra, Accept &&accept,
                    OnSeg &&on_seg, std::vector<int> &K, std::vector<Seg> &segs, StripList &sl,
-                   std::vector<int> &strip_al) {
+                   std::vector<int> &strip_al, int kpad = 1) {
     RowStrips rows(s);
     for (int al = 0; al < s.nr; ++al)
         if (s.x_of_r[al] >= 0) rows.get(s, al);  // filled here: read-only in the parallel phases
@@ -1130,7 +1131,7 @@ double column_strips(const Site &s, const TLay &t, const ColProg &cp, bool skip_
             for (auto &c : cs[k]) {
                 const std::vector<std::pair<int, int>> &rs = rows.of[c.sg.al];
                 c.sg.koff = K[c.sg.al];
-                K[c.sg.al] += s.rsize(c.sg.ar);
+                K[c.sg.al] += ceil_div(s.rsize(c.sg.ar), kpad) * kpad;
                 c.strip0 = strip_n;
                 c.src0 = src_n;
                 strip_n += (int64_t)rs.size();
@@ -1169,6 +1170,94 @@ double column_strips(const Site &s, const TLay &t, const ColProg &cp, bool skip_
             8, 1);
     }
     return extra_sum;
+}
+
+// Moves a sigma plan's single-source strips into its gather lists (HostPlan::gather): the
+// segments' K offsets are multiples of four, their strips follow one another in segs'
+// order.
+void gather_strips(const Site &s, const std::vector<Seg> &segs, const std::vector<int> &K, HostPlan &P) {
+    RowStrips rows(s);
+    Gather &G = P.gather;
+    StripList out;
+    std::vector<int64_t> q0(s.nr, 0), r0(s.nr, 0);
+    int64_t nq = 0;
+    for (auto &xb : s.X.blk) {
+        const int al = s.ri.get(xb.c);
+        q0[al] = nq;
+        nq += K[al] / 4;
+        r0[al] = (int64_t)G.row.size();
+        const auto &rs = rows.get(s, al);
+        int next = 0;
+        for (size_t k = 0; k < rs.size(); ++k) {
+            if (rs[k].first != next) throw std::runtime_error("row strips do not cover the output block");
+            for (int r = 0; r < rs[k].second; ++r) G.row.push_back({(int)k, r, rs[k].second, 0});
+            next += rs[k].second;
+        }
+        if (next != xb.rows) throw std::runtime_error("row strips do not cover the output block");
+    }
+    const TaskVec<Strip> &st = P.wapply.strips;
+    G.src.resize(st.size());
+    G.quad.resize((size_t)nq);
+    // strips that stay, per segment: counted, then written at their places
+    std::vector<int64_t> first(segs.size() + 1, 0), nst(segs.size() + 1, 0), nsr(segs.size() + 1, 0),
+        el(segs.size() + 1, 0);
+    for (size_t i = 0; i < segs.size(); ++i) first[i + 1] = first[i] + (int64_t)rows.of[segs[i].al].size();
+    if (first.back() != (int64_t)st.size() || first.back() > INT32_MAX)
+        throw std::runtime_error("W-application strips out of step with their segments");
+    auto single = [&](const Strip &x) {
+        return x.s1 - x.s0 < 2 && (x.s1 == x.s0 || P.wapply.srcs[x.s0].ld == x.rows);
+    };
+    parallel_for((int)segs.size(), [&](int i) {
+        for (int64_t k = first[i]; k < first[i + 1]; ++k) {
+            if (single(st[k])) continue;
+            ++nst[i + 1];
+            nsr[i + 1] += st[k].s1 - st[k].s0;
+            el[i + 1] += (int64_t)st[k].rows * st[k].cols;
+        }
+    });
+    for (size_t i = 0; i < segs.size(); ++i) {
+        nst[i + 1] += nst[i];
+        nsr[i + 1] += nsr[i];
+        el[i + 1] += el[i];
+    }
+    out.strips.resize((size_t)nst.back());
+    out.srcs.resize((size_t)nsr.back());
+    std::vector<double> read(segs.size(), 0.0);
+    parallel_for((int)segs.size(), [&](int i) {
+        const Seg &sg = segs[i];
+        const int rsz = s.rsize(sg.ar);
+        int64_t a = nst[i], b = nsr[i], dst = P.n_t + el[i];
+        for (int64_t k = first[i]; k < first[i + 1]; ++k) {
+            const Strip &x = st[k];
+            if (x.s1 > x.s0) read[i] += (double)x.rows * x.cols;
+            if (single(x)) {
+                if (x.s1 == x.s0) G.src[k] = {-1, 0.0};
+                else G.src[k] = {P.wapply.srcs[x.s0].off, P.wapply.srcs[x.s0].coef};
+                continue;
+            }
+            G.src[k] = {dst, 1.0};
+            out.strips[a++] = {dst, x.rows, x.cols, x.rows, (int)b, (int)b + x.s1 - x.s0};
+            for (int q = x.s0; q < x.s1; ++q) out.srcs[b++] = P.wapply.srcs[q];
+            dst += (int64_t)x.rows * x.cols;
+        }
+        for (int k = 0; k < rsz; k += 4)
+            G.quad[q0[sg.al] + (sg.koff + k) / 4] = {(int)first[i], 8 * k + std::min(4, rsz - k)};
+    });
+    for (double r : read) G.elements += r;
+    for (auto &g : P.g2.groups) {  // c is the al block's offset in sigma
+        for (auto &xb : s.X.blk)
+            if (xb.off == g.c && xb.rows == g.M) {
+                const int al = s.ri.get(xb.c);
+                g.a = 0;
+                g.gq = q0[al];
+                g.grow = r0[al];
+            }
+    }
+    P.wapply.strips.swap(out.strips);
+    P.wapply.srcs.swap(out.srcs);
+    P.gathered = true;
+    P.n_t += el.back();  // one arena: T, then the strips that stay
+    P.n_c = 0;
 }
 
 void patch_strips(StripList &sl, const std::vector<int> &strip_al, const std::vector<int64_t> &c_off) {
@@ -1257,7 +1346,7 @@ GemmList batch_gemm(const GemmList &gl, int nvec, int64_t a_step, int64_t b_step
 
 // ============================================================ sigma
 HostPlan build_sigma_plan(const mq_site_desc &d, int tm, int tn, int kc, FuseRule fuse, bool ref_count,
-                          int schedule) {
+                          int schedule, bool gather) {
     if (schedule == SCHED_REFERENCE && d.symm == MQ_SYMM_SU2U1) {
         Mpo w = to_mpo(d.mpo);
         if ((w.rows - w.one_rows) >= (w.cols - w.one_cols)) return build_sigma_plan_rbtm(d, tm, tn, kc, ref_count);
@@ -1290,7 +1379,7 @@ HostPlan build_sigma_plan(const mq_site_desc &d, int tm, int tn, int kc, FuseRul
             return r_operand(s, R, sg.b2, s.right.q[sg.ar], s.right.q[sg.al], &sg.rblk, &sg.rtrans, &sg.rscale);
         },
         [&](const Seg &sg) { ref_trim += 2.0 * s.X.blk[s.x_of_r[sg.al]].rows * s.rsize(sg.ar) * s.rsize(sg.al); }, K,
-        segs, P.wapply, strip_al);
+        segs, P.wapply, strip_al, gather ? 4 : 1);
     std::vector<int64_t> c_off(s.nr, 0), rb_off(s.nr, 0);
     int64_t ct = 0, rbt = 0;
     for (auto &xb : s.X.blk) {
@@ -1348,6 +1437,7 @@ HostPlan build_sigma_plan(const mq_site_desc &d, int tm, int tn, int kc, FuseRul
     }
     P.exec_flops = P.g1.flops() + P.g2.flops();
     for (auto &st : P.wapply.strips) P.exec_flops += 2.0 * st.rows * st.cols * (st.s1 - st.s0);
+    if (gather) gather_strips(s, segs, K, P);
     if (!ref_count) {
         P.ref_flops = -1;
     } else if (ref_lbtm) {

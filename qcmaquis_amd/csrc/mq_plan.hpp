@@ -73,6 +73,8 @@ struct GemmGroup {
     int kchunk;
     int tm, tn;
     int64_t rowmap;
+    // gathered A operand (see Gather): first entries of the group in quads and rows
+    int64_t gq, grow;
 };
 struct RowMap {
     int64_t off;  // relative to the group's c
@@ -135,6 +137,29 @@ struct StripList {
     TaskVec<Src> srcs;
     std::vector<Pack> packs;
 };
+// The A operand of a sigma's output GEMM, read from where it lies instead of from a C
+// panel: row block `strip` (one |lb| range of the output block's rows) of K segment `seg`
+// (one MPO column and right charge) is one T block times a coefficient, or nothing, or a
+// sum that the W application wrote.  K is cut into quads of four columns of one
+// segment; the last quad of a segment is partly empty, and the rows of RB it meets are zero.
+struct GatherSrc {  // [seg's desc + strip]
+    int64_t off;    // -1: zero
+    double coef;
+};
+struct GatherQuad {  // [gq + k / 4]
+    int desc;   // of its segment
+    int k0len;  // 8 * first column in the segment + columns (1..4)
+};
+struct GatherRow {  // [grow + row of the output block]
+    int strip, row, ld, pad;
+};
+struct Gather {
+    TaskVec<GatherSrc> src;
+    TaskVec<GatherQuad> quad;
+    std::vector<GatherRow> row;
+    double elements = 0;  // T and C elements the GEMM reads
+};
+
 // (re)compute the packs of a strip list, keeping the strip order
 void make_packs(StripList &sl);
 
@@ -156,6 +181,10 @@ struct HostPlan {
     GemmList g1;                // T = LA * PRP    (sigma, lstep) ; t = X * RC (rstep)
     StripList wapply;           // T -> C          / t -> BUF
     GemmList g2;                // y = C * RB      / tmp = C^T X  / tmp = BUF * PRP^T
+    // sigma plans built for the device (lbtm form): g2 reads its A operand through
+    // `gather` from one arena, T followed by the C strips that wapply still writes
+    bool gathered = false;
+    Gather gather;
     std::vector<Copy2D> scatter;  // tmp -> output boundary (steps)
     // output boundary structure (steps)
     int out_aux = 0;
@@ -187,8 +216,11 @@ struct FuseRule {
 // rbtm (build_sigma_plan_rbtm, no fused rows) where (rows - one_rows) >=
 // (cols - one_cols) for SU2U1, lbtm elsewhere.
 enum SigmaSchedule { SCHED_LBTM = 0, SCHED_REFERENCE = 1 };
+// gather: the lbtm form's output GEMM reads T through HostPlan::gather, and only the
+// strips of several sources stay in wapply (their dst counts from T's start); without it
+// every strip is written to C, the form the task lists are checked in.
 HostPlan build_sigma_plan(const mq_site_desc &d, int tile_m, int tile_n, int kchunk_target, FuseRule fuse = {},
-                          bool ref_count = true, int schedule = SCHED_LBTM);
+                          bool ref_count = true, int schedule = SCHED_LBTM, bool gather = false);
 // The rbtm schedule (site_hamil.hpp:149-204) on every site: t = X * RC, the rbtm
 // W application into BUF, S = LA^T * BUF, y = S reshaped to the left-paired layout.
 HostPlan build_sigma_plan_rbtm(const mq_site_desc &d, int tile_m, int tile_n, int kchunk_target,

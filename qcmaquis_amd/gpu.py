@@ -99,28 +99,33 @@ COPY2D = np.dtype([("dst", "<i8"), ("src", "<i8"), ("rows", "<i4"), ("cols", "<i
 GEMMGROUP = np.dtype([("a", "<i8"), ("b", "<i8"), ("c", "<i8"), ("part", "<i8"), ("M", "<i4"), ("N", "<i4"),
                       ("K", "<i4"), ("lda", "<i4"), ("ldb", "<i4"), ("ldc", "<i4"), ("transA", "<i4"),
                       ("transB", "<i4"), ("split", "<i4"), ("kchunk", "<i4"), ("tm", "<i4"), ("tn", "<i4"),
-                      ("rowmap", "<i8")], align=True)
+                      ("rowmap", "<i8"), ("gq", "<i8"), ("grow", "<i8")], align=True)
 ROWMAP = np.dtype([("off", "<i8"), ("ld", "<i4"), ("pad", "<i4")], align=True)
 GEMMTILE = np.dtype([("g", "<i4"), ("mt", "<i4"), ("nt", "<i4"), ("ks", "<i4")], align=True)
 STRIP = np.dtype([("dst", "<i8"), ("rows", "<i4"), ("cols", "<i4"), ("ldd", "<i4"), ("s0", "<i4"),
                   ("s1", "<i4")], align=True)
 SRC = np.dtype([("off", "<i8"), ("ld", "<i4"), ("coef", "<f8")], align=True)
+GATHERSRC = np.dtype([("off", "<i8"), ("coef", "<f8")])
+GATHERQUAD = np.dtype([("desc", "<i4"), ("k0len", "<i4")])
+GATHERROW = np.dtype([("strip", "<i4"), ("row", "<i4"), ("ld", "<i4"), ("pad", "<i4")])
 PART_DTYPES = [COPY2D, COPY2D, COPY2D, GEMMGROUP, GEMMTILE, STRIP, SRC, GEMMGROUP, GEMMTILE, COPY2D, STRIP, SRC,
-               ROWMAP, ROWMAP, np.dtype(np.uint8)]
+               ROWMAP, ROWMAP, np.dtype(np.uint8), GATHERSRC, GATHERQUAD, GATHERROW]
 PART_NAMES = ["arrL", "arrR", "reshape", "g1_groups", "g1_tiles", "strips", "srcs", "g2_groups", "g2_tiles",
-              "scatter", "comb_strips", "comb_srcs", "g1_rowmap", "g2_rowmap", "live"]
+              "scatter", "comb_strips", "comb_srcs", "g1_rowmap", "g2_rowmap", "live",
+              "gather_srcs", "gather_quads", "gather_rows"]
 KIND = {"sigma": 0, "lstep": 1, "rstep": 2, "diag": 3}
 
 
 class HostPlan:
     """Task lists of a plan, built on the host (no GPU needed)."""
 
-    def __init__(self, site: SiteDesc, kind: str, fuse=1, fuse_ratio=0, fuse_min=0, schedule=0):
-        """schedule 1: sigma plans take the reference's per-site choice of lbtm or
+    def __init__(self, site: SiteDesc, kind: str, fuse=1, fuse_ratio=0, fuse_min=0, schedule=0, gather=False):
+        """gather: a sigma plan in the form the device runs, its output GEMM's operand
+        gathered (MQ_HOST_GATHER).  schedule 1: sigma plans take the reference's per-site choice of lbtm or
         rbtm (MQ_HOST_SCHED_REFERENCE); self.rbtm tells which was built."""
         L = lib()
         h = C.c_void_p()
-        code = KIND[kind] | ((fuse + 1) << 8) | (fuse_ratio << 10) | (fuse_min << 18) | ((schedule & 1) << 30)
+        code = KIND[kind] | ((fuse + 1) << 8) | (fuse_ratio << 10) | (fuse_min << 18) | ((schedule & 1) << 30) | (16 if gather else 0)
         if L.mq_host_plan_create(site.ptr(), code, C.byref(h)) != 0:
             raise MQError(L.mq_host_last_error().decode())
         try:
