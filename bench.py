@@ -82,7 +82,7 @@ def sigma_kernels(form):
     t = "double" if form == "fp64" else "float"
     x3 = "true" if form == "bf16x3" else "false"
     return {"reshape": f"k_copy2d<0, double, {t}>", "gemm_T": f"k_gemm<0, {t}, {t}, {x3}>",
-            "w_apply": f"k_wapply<0, {t}, false>", "gemm_out": f"k_gemm<1, {t}, double, {x3}>",
+            "w_apply": f"k_wapply<0, {t}, false>", "gemm_out": f"k_gemm_gather<{t}, {x3}>",
             "split_reduce": f"k_split_reduce<1, {t}, double>"}
 
 

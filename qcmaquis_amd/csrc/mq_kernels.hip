@@ -323,7 +323,10 @@ __device__ __forceinline__ void gemm_fetch_b(const GemmGroup &g, const T *__rest
         if constexpr (GATHER) {
             const int gn = n0 + j, gk = k0 + k;
             T v = 0;
-            if (gn < g.N && gk < kend) v = B[g.b + gk + (int64_t)gn * g.ldb];
+            // (transB is never set here; tested, it keeps the compiler from holding every
+            // column's address in registers, which spills 42 in the BF16x3 body)
+            if (gn < g.N && gk < kend)
+                v = g.transB ? B[g.b + gn + (int64_t)gk * g.ldb] : B[g.b + gk + (int64_t)gn * g.ldb];
             st.b[r] = v;
         } else {
             const int gn = min(n0 + j, g.N - 1), gk = min(k0 + k, kend - 1);
