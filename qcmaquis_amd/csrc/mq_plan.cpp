@@ -242,16 +242,21 @@ int column_tile(int N) {
     return best;
 }
 
-void add_gemm(GemmList &gl, GemmGroup g, int tm, int tn, int kchunk_target) {
-    if (g.rowmap < 0 || (g.rowmap > 0 && g.rowmap - 1 + g.M > (int64_t)gl.rowmap.size()))
-        throw std::runtime_error("GEMM row map out of range");
+// a group's tile shape; 0: automatic (128 rows unless M fits 64; the column tile of
+// column_tile)
+void tile_shape(GemmGroup &g, int tm, int tn) {
     if ((tm != 0 && tm != 64 && tm != 128) || (tn != 0 && (tn < 16 || tn > 128 || tn % 16)))
         throw std::runtime_error("GEMM tile shape out of range");
-    g.split = 1;
-    g.kchunk = std::max(g.K, 1);
-    // 0: automatic (128 rows unless M fits 64; the column tile of column_tile)
     g.tm = tm ? tm : (g.M > 64 ? 128 : 64);
     g.tn = tn ? tn : column_tile(g.N);
+}
+
+// Appends a group of known tile shape with its tiles.
+void add_tiles(GemmList &gl, GemmGroup g, int kchunk_target) {
+    if (g.rowmap < 0 || (g.rowmap > 0 && g.rowmap - 1 + g.M > (int64_t)gl.rowmap.size()))
+        throw std::runtime_error("GEMM row map out of range");
+    g.split = 1;
+    g.kchunk = std::max(g.K, 1);
     if (g.M == 0 || g.N == 0) return;
     int mt = ceil_div(g.M, g.tm), nt = ceil_div(g.N, g.tn);
     // split K when the output is small and K long: chunks of about kchunk_target
@@ -280,7 +285,8 @@ void add_gemm(GemmList &gl, GemmGroup g, int tm, int tn, int kchunk_target) {
     }
 }
 
-// The tiles of a plan's GEMM list, once every group is in it.  A launch whose K loops
+// The tiles of a plan's GEMM list, once every group is in it (push_back; the groups have no
+// tiles until then).  A launch whose K loops
 // add up to less than kFillTiles chunks of kchunk_target would leave most of the 256
 // CUs idle behind a few long K loops (each K step is one exposed round trip of about
 // 0.2 us), so the chunk shrinks until the launch has about kFillTiles tiles, down to
@@ -290,15 +296,17 @@ void add_gemm(GemmList &gl, GemmGroup g, int tm, int tn, int kchunk_target) {
 // per CU; the L=24 m=512 centre has 1,362 at the default chunk and is not touched.
 constexpr int kFillTiles = 1024, kMinChunk = 128;
 void finish_gemm(GemmList &gl, int tm, int tn, int kchunk_target) {
-    int64_t total = 0;  // K steps of every output tile
-    for (auto &g : gl.groups) total += (int64_t)ceil_div(g.M, g.tm) * ceil_div(g.N, g.tn) * g.K;
-    const int64_t fill = (total / kFillTiles + 15) / 16 * 16;
-    const int chunk = (int)std::min<int64_t>(kchunk_target, std::max<int64_t>(kMinChunk, fill));
     std::vector<GemmGroup> groups;
     groups.swap(gl.groups);
-    gl.tiles.clear();
-    gl.ws = 0;
-    for (auto &g : groups) add_gemm(gl, g, tm, tn, chunk);
+    gl.groups.reserve(groups.size());
+    int64_t total = 0;  // K steps of every output tile
+    for (auto &g : groups) {
+        tile_shape(g, tm, tn);
+        total += (int64_t)ceil_div(g.M, g.tm) * ceil_div(g.N, g.tn) * g.K;
+    }
+    const int64_t fill = (total / kFillTiles + 15) / 16 * 16;
+    const int chunk = (int)std::min<int64_t>(kchunk_target, std::max<int64_t>(kMinChunk, fill));
+    for (auto &g : groups) add_tiles(gl, g, chunk);
     order_tiles(gl);
 }
 
@@ -574,7 +582,7 @@ struct TLay {
 // psi's rows of those chunks, packed into the psi arena by the reshape.  The
 // combination strips (comb) build the panels from the arranged rows.
 TLay t_layout(const Site &s, const BLayout &L, PRP &prp, ColProg *cp, std::vector<Copy2D> *arr,
-              std::vector<Copy2D> *reshape, StripList *comb, GemmList *g1, int tm, int tn, int kc) {
+              std::vector<Copy2D> *reshape, StripList *comb, GemmList *g1) {
     struct A {
         int lb, lk;
         const BBlk *blk;
@@ -676,7 +684,7 @@ TLay t_layout(const Site &s, const BLayout &L, PRP &prp, ColProg *cp, std::vecto
             g.ldb = g.K;
             g.ldc = g.M;
             g.rowmap = map0[lk] + 1;
-            add_gemm(*g1, g, tm, tn, kc);
+            g1->groups.push_back(g);
         }
     }
     if (!cp || cp->fo.empty()) return t;
@@ -909,7 +917,7 @@ TLay t_layout(const Site &s, const BLayout &L, PRP &prp, ColProg *cp, std::vecto
         g.ldb = pn.K;
         g.ldc = pn.rows;
         g.rowmap = map0[k] + 1;
-        add_gemm(*g1, g, tm, tn, kc);
+        g1->groups.push_back(g);
     }
     return t;
 }
@@ -1266,7 +1274,10 @@ void patch_strips(StripList &sl, const std::vector<int> &strip_al, const std::ve
 
 }  // namespace
 
-void tile_gemm(GemmList &gl, GemmGroup g, int tm, int tn, int kc) { add_gemm(gl, g, tm, tn, kc); }
+void tile_gemm(GemmList &gl, GemmGroup g, int tm, int tn, int kc) {
+    tile_shape(g, tm, tn);
+    add_tiles(gl, g, kc);
+}
 
 void order_tiles(GemmList &gl) {
     std::vector<GemmTile> t;
@@ -1360,7 +1371,7 @@ HostPlan build_sigma_plan(const mq_site_desc &d, int tm, int tn, int kc, FuseRul
     P.vec_len = s.X.total;
     PRP prp = prp_layout(s, P.reshape);
     ColProg cp = column_program(s, false, fuse);
-    TLay t = t_layout(s, L, prp, &cp, &P.arrL, &P.reshape, &P.combL, &P.g1, tm, tn, kc);
+    TLay t = t_layout(s, L, prp, &cp, &P.arrL, &P.reshape, &P.combL, &P.g1);
     P.n_prp = prp.total;
     P.n_la = t.la_total;
     P.n_t = t.t_total;
@@ -1371,7 +1382,7 @@ HostPlan build_sigma_plan(const mq_site_desc &d, int tm, int tn, int kc, FuseRul
     const bool ref_lbtm =
         ref_count && (s.symm != MQ_SYMM_SU2U1 || (s.W.rows - s.W.one_rows) < (s.W.cols - s.W.one_cols));
     TLay tall;
-    if (ref_lbtm) tall = t_layout(s, L, prp, nullptr, nullptr, nullptr, nullptr, nullptr, tm, tn, kc);
+    if (ref_lbtm) tall = t_layout(s, L, prp, nullptr, nullptr, nullptr, nullptr, nullptr);
     double ref_axpy = 0, ref_trim = 0;
     ref_axpy = column_strips(
         s, t, cp, false, [&](int b2) { return ref_lbtm ? reference_axpy_flops(s, tall, b2) : 0.0; },
@@ -1433,7 +1444,7 @@ HostPlan build_sigma_plan(const mq_site_desc &d, int tm, int tn, int kc, FuseRul
         g.lda = xb.rows;
         g.ldb = std::max(K[r], 1);
         g.ldc = xb.rows;
-        add_gemm(P.g2, g, tm, tn, kc);
+        P.g2.groups.push_back(g);
     }
     P.exec_flops = P.g1.flops() + P.g2.flops();
     for (auto &st : P.wapply.strips) P.exec_flops += 2.0 * st.rows * st.cols * (st.s1 - st.s0);
@@ -1464,10 +1475,10 @@ HostPlan build_lstep_plan(const mq_site_desc &d, int tm, int tn, int kc, FuseRul
     P.vec_len = s.X.total;
     PRP prp = prp_layout(s, P.reshape);
     ColProg cp = column_program(s, true, fuse);
-    TLay t = t_layout(s, L, prp, &cp, &P.arrL, &P.reshape, &P.combL, &P.g1, tm, tn, kc);
+    TLay t = t_layout(s, L, prp, &cp, &P.arrL, &P.reshape, &P.combL, &P.g1);
     P.n_prp = prp.total;
     TLay tall;
-    if (ref_count) tall = t_layout(s, L, prp, nullptr, nullptr, nullptr, nullptr, nullptr, tm, tn, kc);
+    if (ref_count) tall = t_layout(s, L, prp, nullptr, nullptr, nullptr, nullptr, nullptr);
     P.n_la = t.la_total;
     P.n_t = t.t_total;
     double axf = 0;
@@ -1507,7 +1518,7 @@ HostPlan build_lstep_plan(const mq_site_desc &d, int tm, int tn, int kc, FuseRul
         g.ldb = xb.rows;
         g.ldc = K[r];
         g.transA = 1;
-        add_gemm(P.g2, g, tm, tn, kc);
+        P.g2.groups.push_back(g);
     }
     // output boundary: per b2, blocks (ar, al) in descending order
     P.out_aux = s.W.cols;
@@ -1578,7 +1589,7 @@ struct RbtmCore {
 // row, hermitian-partner rows included; a (b1, ol, or) group only when L[b1] has
 // the block (ket ol, bra or), as rbtm_axpy_gemm skips the others); otherwise the
 // right step (rows whose output boundary slice is stored).
-RbtmCore rbtm_core(const Site &s, const BLayout &R, const BLayout *Lsig, HostPlan &P, int tm, int tn, int kc) {
+RbtmCore rbtm_core(const Site &s, const BLayout &R, const BLayout *Lsig, HostPlan &P) {
     RbtmCore out;
     // MPSBoundaryProduct: t[b2] = X * Rop[b2] right-trimmed to X's right charges;
     // RC_c stacks Rop[b2](c, c') horizontally over (b2, c').
@@ -1637,7 +1648,7 @@ RbtmCore rbtm_core(const Site &s, const BLayout &R, const BLayout *Lsig, HostPla
         g.lda = xb.rows;
         g.ldb = xb.cols;
         g.ldc = xb.rows;
-        add_gemm(P.g1, g, tm, tn, kc);
+        P.g1.groups.push_back(g);
     }
     // rbtm tasks (apply_op.hpp:114-209): buf[b1](ol, or) += coef * t rows.  Per b1: raw list
     // keyed by (or, ol, col0), BUF_or stacks rows over (b1, ol).
@@ -1816,7 +1827,7 @@ HostPlan build_rstep_plan(const mq_site_desc &d, int tm, int tn, int kc) {
     P.vec_len = s.X.total;
     PRP prp = prp_layout(s, P.reshape);
     P.n_prp = prp.total;
-    RbtmCore core = rbtm_core(s, R, nullptr, P, tm, tn, kc);
+    RbtmCore core = rbtm_core(s, R, nullptr, P);
     const std::vector<int> &Mr = core.Mr;
     const std::vector<RowBlk> &rowblks = core.rowblks;
     const std::vector<int64_t> &buf_off = core.buf_off;
@@ -1842,7 +1853,7 @@ HostPlan build_rstep_plan(const mq_site_desc &d, int tm, int tn, int kc) {
         g.ldb = s.lsize(l);
         g.ldc = Mr[l];
         g.transB = 1;
-        add_gemm(P.g2, g, tm, tn, kc);
+        P.g2.groups.push_back(g);
     }
     P.out_aux = s.W.rows;
     std::vector<std::vector<const RowBlk *>> per_b1(s.W.rows);
@@ -1906,7 +1917,7 @@ HostPlan build_sigma_plan_rbtm(const mq_site_desc &d, int tm, int tn, int kc, bo
     P.vec_len = s.X.total;
     for (auto &xb : s.X.blk) P.reshape.push_back(mk_copy(xb.off, xb.off, xb.rows, xb.cols, xb.rows, xb.rows, false, 1.0));
     P.n_prp = s.X.total;
-    RbtmCore core = rbtm_core(s, R, &L, P, tm, tn, kc);
+    RbtmCore core = rbtm_core(s, R, &L, P);
     // LA_or (K_or x |or|, leading dimension K_or = Mr[or]): row block rb.row holds
     // L[b1](ol, or) (ket rows, bra columns), or for a hermitian-partner row the
     // stored block (or, ol) of L[conj(b1)] transposed, scaled by the conjugate
@@ -1947,7 +1958,7 @@ HostPlan build_sigma_plan_rbtm(const mq_site_desc &d, int tm, int tn, int kc, bo
         g.ldb = std::max(core.Mr[l], 1);
         g.ldc = s.lsize(l);
         g.transA = 1;
-        add_gemm(P.g2, g, tm, tn, kc);
+        P.g2.groups.push_back(g);
     }
     // right-paired S -> left-paired y: the inverse of the psi reshape (prp_layout)
     for (auto &xb : s.X.blk) {
@@ -2020,7 +2031,7 @@ double reference_sigma_flops(const mq_site_desc &d) {
     bool lbtm = s.symm != MQ_SYMM_SU2U1 || (s.W.rows - s.W.one_rows) < (s.W.cols - s.W.one_cols);
     double f = 0;
     if (lbtm) {
-        TLay t = t_layout(s, L, prp, nullptr, nullptr, nullptr, nullptr, nullptr, 64, 64, 1 << 30);
+        TLay t = t_layout(s, L, prp, nullptr, nullptr, nullptr, nullptr, nullptr);
         f += t.gemm_flops;
         std::vector<Raw> raw;
         for (int b2 = 0; b2 < s.W.cols; ++b2) {
@@ -2254,7 +2265,7 @@ HostPlan build_diag_plan(const mq_site_desc &d, int tm, int tn, int kc) {
             g.lda = ls;
             g.ldb = std::max(K, 1);
             g.ldc = xb.rows;
-            add_gemm(P.g2, g, tm, tn, kc);
+            P.g2.groups.push_back(g);
         }
     }
     finish_gemm(P.g2, tm, tn, kc);
