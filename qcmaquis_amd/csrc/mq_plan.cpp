@@ -16,7 +16,6 @@
 #include <atomic>
 #include <cstdlib>
 #include <exception>
-#include <map>
 #include <mutex>
 #include <new>
 #include <thread>
@@ -445,6 +444,7 @@ struct FRow {  // the |lb| rows of one output (lb, al) and one right charge ar
     int lb, al, ar;
     int panel, row;
     int64_t tf;  // T-arena offset of its T block (stored contiguously, leading dimension |lb|)
+    uint64_t hash;  // of ar and the chunks' input states: the panel's key
     std::vector<FChunk> chunk;
 };
 struct FOut {  // output state `col` of physical block pout in column b2
@@ -591,6 +591,8 @@ TLay t_layout(const Site &s, const BLayout &L, PRP &prp, ColProg *cp, std::vecto
         int row;
     };
     const int nb1 = s.W.rows;
+    // row maps are filled by one thread per 16,384 rows (about its own start, 20 us)
+    auto map_grain = [](int64_t n, int64_t rows) { return (int)std::max<int64_t>(1, n * 16384 / std::max<int64_t>(rows, 1)); };
     TLay t;
     t.M.assign(s.nl, 0);
     t.Mtot.assign(s.nl, 0);
@@ -670,7 +672,7 @@ TLay t_layout(const Site &s, const BLayout &L, PRP &prp, ColProg *cp, std::vecto
                 for (int r = 0; r < t.M[lk]; ++r)
                     if (rm[r].off < 0) throw std::runtime_error("T panel row without a block");
             },
-            1, 1);
+            map_grain(s.nl, map0[s.nl] - map0[0]), 1);
         for (int lk = 0; lk < s.nl; ++lk) {
             if (t.M[lk] == 0) continue;
             GemmGroup g{};
@@ -703,8 +705,8 @@ TLay t_layout(const Site &s, const BLayout &L, PRP &prp, ColProg *cp, std::vecto
     const int ng = (int)cp->fo.size();
     // coupling of class c of input `in` at (lk, lb); zero where the charges or spins do not
     // let the block contribute
-    auto factor = [&](const FOut &o, const FIn &in, const FCls &c, int lk, int lb, int ar, int al) {
-        if (!s.su2) return 1.0;
+    // (SU(2) only: it is 1 in the abelian symmetry)
+    auto factor = [&](const FOut &o, const FCls &c, int lk, int lb, int ar, int al) {
         const int ap = s.W.rspin[o.b2];
         const int i = spin2(s.left.q[lb]), j = spin2(s.left.q[lk]);
         const int jp = spin2(s.right.q[ar]), ip = spin2(s.right.q[al]);
@@ -719,16 +721,29 @@ TLay t_layout(const Site &s, const BLayout &L, PRP &prp, ColProg *cp, std::vecto
         const int al = s.lp_r[(size_t)lb * s.np + o.pout];
         return al >= 0 && s.x_of_r[al] >= 0 ? al : -1;
     };
-    // f(in index, block, coefficient) for every source of output o: each L block of each
-    // member row, the entries of one row summed; blocks whose every coupling vanishes
-    // are left out
-    auto for_sources = [&](const FOut &o, auto &&f) {
-        thread_local std::vector<double> tab;  // [class][lk][lb]
+    // The sources of output o: each L block of each member row, the entries of one row
+    // summed; blocks whose every coupling vanishes are left out.
+    struct FSrc {
+        int at;   // [lb][in][lk]
+        int row;  // LA row of the block
+        double c;
+    };
+    auto list_sources = [&](const FOut &o, TaskVec<FSrc> &out) {
+        thread_local std::vector<double> tab;  // coupling [class][lk][lb], of SU(2)
         thread_local std::vector<char> have;
-        for (size_t q = 0; q < o.in.size(); ++q) {
+        const int ni = (int)o.in.size();
+        size_t most = 0;
+        for (auto &in : o.in)
+            for (size_t m = 0; m < in.mem.size(); ++m)
+                if (m == 0 || in.mem[m].b1 != in.mem[m - 1].b1) most += blk[in.mem[m].b1].size();
+        out.resize(most);
+        size_t n = 0;
+        for (int q = 0; q < ni; ++q) {
             const FIn &in = o.in[q];
-            tab.assign(in.cls.size() * nl * nl, 0.0);
-            have.assign(in.cls.size() * nl * nl, 0);
+            if (s.su2) {
+                tab.resize(in.cls.size() * nl * nl);
+                have.assign(in.cls.size() * nl * nl, 0);
+            }
             for (size_t m0 = 0; m0 < in.mem.size();) {
                 size_t m1 = m0;
                 while (m1 < in.mem.size() && in.mem[m1].b1 == in.mem[m0].b1) ++m1;
@@ -736,31 +751,48 @@ TLay t_layout(const Site &s, const BLayout &L, PRP &prp, ColProg *cp, std::vecto
                     const int ar = right_in(in, a.lk), al = right_out(o, a.lb);
                     if (ar < 0 || al < 0) continue;
                     double c = 0.0;
-                    bool any = false;
+                    bool any = !s.su2;
                     for (size_t m = m0; m < m1; ++m) {
+                        if (!s.su2) {
+                            c += in.mem[m].w;
+                            continue;
+                        }
                         const size_t at = ((size_t)in.mem[m].cls * nl + a.lk) * nl + a.lb;
                         if (!have[at]) {
-                            tab[at] = factor(o, in, in.cls[in.mem[m].cls], a.lk, a.lb, ar, al);
+                            tab[at] = factor(o, in.cls[in.mem[m].cls], a.lk, a.lb, ar, al);
                             have[at] = 1;
                         }
                         any = any || tab[at] != 0.0;
                         c += in.mem[m].w * tab[at];
                     }
-                    if (any) f((int)q, a, c);
+                    if (any) out[n++] = {(a.lb * ni + q) * nl + a.lk, a.row, c};
                 }
                 m0 = m1;
             }
         }
+        out.resize(n);
     };
-    // 1. (parallel) the rows of each output and their chunks, with source counts
+    // 1. (parallel) the sources of each output, its rows and their chunks.  The sources are
+    // kept for step 4: listing them is the larger part of both steps.
+    std::vector<TaskVec<FSrc>> srcs(ng);
+    // a thread is worth starting (some 20 us) for about 4,096 sources; estimated from the
+    // entries and the blocks per MPO row
+    double work = 1.0;
+    for (auto &o : cp->fo)
+        for (auto &in : o.in) work += (double)in.mem.size();
+    size_t nblk = 0;
+    for (auto &b : blk) nblk += b.size();
+    work *= (double)nblk / std::max(nb1, 1);
+    const int grain = (int)std::min(1e9, std::max(4.0, ng * 4096.0 / work));
     parallel_for(
         ng,
         [&](int gi) {
             FOut &o = cp->fo[gi];
             thread_local std::vector<int> cnt;  // [lb][in][lk]
             const size_t ni = o.in.size();
+            list_sources(o, srcs[gi]);
             cnt.assign(ni * nl * nl, 0);
-            for_sources(o, [&](int q, const A &a, double) { ++cnt[((size_t)a.lb * ni + q) * nl + a.lk]; });
+            for (auto &x : srcs[gi]) ++cnt[x.at];
             for (int lb = 0; lb < nl; ++lb) {
                 const int al = right_out(o, lb);
                 if (al < 0) continue;
@@ -772,33 +804,44 @@ TLay t_layout(const Site &s, const BLayout &L, PRP &prp, ColProg *cp, std::vecto
                         const int ar = right_in(o.in[q], lk);
                         size_t r = r0;
                         while (r < o.rows.size() && o.rows[r].ar != ar) ++r;
-                        if (r == o.rows.size()) o.rows.push_back({lb, al, ar, 0, 0, 0, {}});
-                        o.rows[r].chunk.push_back({(int)q, lk, n});
+                        if (r == o.rows.size()) o.rows.push_back({lb, al, ar, 0, 0, 0, (uint64_t)ar, {}});
+                        FRow &row = o.rows[r];
+                        row.chunk.push_back({(int)q, lk, n});
+                        // (FNV-1a over the panel's key)
+                        row.hash = (row.hash ^ (uint64_t)(o.in[q].pin * 256 + o.in[q].row)) * 1099511628211ull;
+                        row.hash = (row.hash ^ (uint64_t)lk) * 1099511628211ull;
                     }
             }
         },
-        4, 1);
+        grain, 1);
     // 2. (sequential) panels keyed by (ar, chunks), rows in output order
-    std::map<std::vector<int>, int> panel_id;
+    std::unordered_multimap<uint64_t, int> panel_of;
     std::vector<Panel> panels;
+    auto same_panel = [&](const Panel &pn, const FOut &o, const FRow &r) {
+        if (pn.ar != r.ar || pn.chunk.size() != r.chunk.size()) return false;
+        for (size_t k = 0; k < r.chunk.size(); ++k) {
+            const FIn &in = o.in[r.chunk[k].in];
+            if (pn.chunk[k] != std::array<int, 3>{in.pin, in.row, r.chunk[k].lk}) return false;
+        }
+        return true;
+    };
     for (auto &o : cp->fo)
         for (auto &r : o.rows) {
-            std::vector<int> key{r.ar};
-            for (auto &c : r.chunk) {
-                key.push_back(o.in[c.in].pin * 256 + o.in[c.in].row);
-                key.push_back(c.lk);
-            }
-            auto it = panel_id.emplace(key, (int)panels.size());
-            if (it.second) {
+            r.panel = -1;
+            for (auto it = panel_of.equal_range(r.hash); it.first != it.second && r.panel < 0; ++it.first)
+                if (same_panel(panels[it.first->second], o, r)) r.panel = it.first->second;
+            if (r.panel < 0) {
+                r.panel = (int)panels.size();
+                panel_of.emplace(r.hash, r.panel);
                 Panel pn;
                 pn.ar = r.ar;
+                pn.chunk.reserve(r.chunk.size());
                 for (auto &c : r.chunk) {
                     pn.chunk.push_back({o.in[c.in].pin, o.in[c.in].row, c.lk});
                     pn.K += s.lsize(c.lk);
                 }
                 panels.push_back(std::move(pn));
             }
-            r.panel = it.first->second;
             Panel &pn = panels[r.panel];
             r.row = pn.rows;
             pn.blocks.push_back({pn.rows, s.lsize(r.lb)});
@@ -843,8 +886,19 @@ TLay t_layout(const Site &s, const BLayout &L, PRP &prp, ColProg *cp, std::vecto
         const size_t s0 = sbase[0];
         comb->strips.resize(sbase[ng]);
         comb->srcs.resize(gbase[ng]);
-        std::vector<uint32_t> comb_key(sbase[ng] - s0);  // lk * nl + lb: strips reading one LA_lk row range run together
-        // 4. (parallel) each output's strips and, in member order, its sources
+        // strips reading one LA_lk row range run together: their places in (lk, lb) order, equal
+        // keys in output order
+        std::vector<size_t> start((size_t)nl * nl + 1, s0);
+        std::vector<size_t> place(sbase[ng] - s0);
+        for (auto &o : cp->fo)
+            for (auto &r : o.rows)
+                for (auto &c : r.chunk) ++start[(size_t)c.lk * nl + r.lb + 1];
+        for (size_t b = 1; b < start.size(); ++b) start[b] += start[b - 1] - s0;
+        size_t *next_place = place.data();
+        for (auto &o : cp->fo)
+            for (auto &r : o.rows)
+                for (auto &c : r.chunk) *next_place++ = start[(size_t)c.lk * nl + r.lb]++;
+        // 4. (parallel) each output's strips and, in their order, its sources
         parallel_for(
             ng,
             [&](int gi) {
@@ -853,12 +907,12 @@ TLay t_layout(const Site &s, const BLayout &L, PRP &prp, ColProg *cp, std::vecto
                 const size_t ni = o.in.size();
                 pos.assign(ni * nl * nl, -1);
                 int base = gbase[gi];
-                size_t st_i = sbase[gi];
+                const size_t *at = place.data() + (sbase[gi] - s0);
                 for (auto &r : o.rows) {
                     const Panel &pn = panels[r.panel];
                     int k = 0;
                     for (auto &c : r.chunk) {
-                        Strip &st = comb->strips[st_i];
+                        Strip &st = comb->strips[*at++];
                         st.dst = pn.lf + r.row + (int64_t)k * pn.rows;
                         st.rows = s.lsize(r.lb);
                         st.cols = s.lsize(c.lk);
@@ -868,22 +922,14 @@ TLay t_layout(const Site &s, const BLayout &L, PRP &prp, ColProg *cp, std::vecto
                         pos[((size_t)r.lb * ni + c.in) * nl + c.lk] = base;
                         base = st.s1;
                         k += s.lsize(c.lk);
-                        comb_key[st_i++ - s0] = (uint32_t)(c.lk * nl + r.lb);
                     }
                 }
-                for_sources(o, [&](int q, const A &a, double c) {
-                    comb->srcs[pos[((size_t)a.lb * ni + q) * nl + a.lk]++] = {t.la_off[a.lk] + a.row, t.Mtot[a.lk], c};
-                });
+                for (auto &x : srcs[gi]) {
+                    const int lk = x.at % nl;
+                    comb->srcs[pos[x.at]++] = {t.la_off[lk] + x.row, t.Mtot[lk], x.c};
+                }
             },
-            4, 1);
-        // stable counting sort by (lk, lb)
-        std::vector<size_t> start((size_t)nl * nl + 1, 0);
-        for (uint32_t k : comb_key) ++start[k + 1];
-        for (size_t b = 1; b < start.size(); ++b) start[b] += start[b - 1];
-        TaskVec<Strip> sorted(comb->strips.size());
-        std::copy_n(comb->strips.begin(), s0, sorted.begin());
-        for (size_t i = 0; i < comb_key.size(); ++i) sorted[s0 + start[comb_key[i]]++] = comb->strips[s0 + i];
-        comb->strips.swap(sorted);
+            grain, 1);
     }
     // row maps of the fused panels: each panel's rows at a known offset, filled in parallel
     std::vector<int64_t> map0(panels.size() + 1, g1 ? (int64_t)g1->rowmap.size() : 0);
@@ -899,7 +945,7 @@ TLay t_layout(const Site &s, const BLayout &L, PRP &prp, ColProg *cp, std::vecto
                 for (auto &rb : pn.blocks)
                     for (int r = 0; r < rb.second; ++r) *rm++ = {(int64_t)rb.first * rsz + r, rb.second, 0};
             },
-            1, 1);
+            map_grain((int64_t)panels.size(), map0.back() - map0[0]), 1);
     }
     for (size_t k = 0; k < panels.size(); ++k) {
         const Panel &pn = panels[k];
@@ -1215,14 +1261,19 @@ void gather_strips(const Site &s, const std::vector<Seg> &segs, const std::vecto
     auto single = [&](const Strip &x) {
         return x.s1 - x.s0 < 2 && (x.s1 == x.s0 || P.wapply.srcs[x.s0].ld == x.rows);
     };
-    parallel_for((int)segs.size(), [&](int i) {
-        for (int64_t k = first[i]; k < first[i + 1]; ++k) {
-            if (single(st[k])) continue;
-            ++nst[i + 1];
-            nsr[i + 1] += st[k].s1 - st[k].s0;
-            el[i + 1] += (int64_t)st[k].rows * st[k].cols;
-        }
-    });
+    // (a few ns per strip: a thread is worth starting for about 16,384 of them)
+    const int grain = (int)std::max<int64_t>(64, (int64_t)segs.size() * 16384 / std::max<int64_t>(first.back(), 1));
+    parallel_for(
+        (int)segs.size(),
+        [&](int i) {
+            for (int64_t k = first[i]; k < first[i + 1]; ++k) {
+                if (single(st[k])) continue;
+                ++nst[i + 1];
+                nsr[i + 1] += st[k].s1 - st[k].s0;
+                el[i + 1] += (int64_t)st[k].rows * st[k].cols;
+            }
+        },
+        grain);
     for (size_t i = 0; i < segs.size(); ++i) {
         nst[i + 1] += nst[i];
         nsr[i + 1] += nsr[i];
@@ -1231,26 +1282,29 @@ void gather_strips(const Site &s, const std::vector<Seg> &segs, const std::vecto
     out.strips.resize((size_t)nst.back());
     out.srcs.resize((size_t)nsr.back());
     std::vector<double> read(segs.size(), 0.0);
-    parallel_for((int)segs.size(), [&](int i) {
-        const Seg &sg = segs[i];
-        const int rsz = s.rsize(sg.ar);
-        int64_t a = nst[i], b = nsr[i], dst = P.n_t + el[i];
-        for (int64_t k = first[i]; k < first[i + 1]; ++k) {
-            const Strip &x = st[k];
-            if (x.s1 > x.s0) read[i] += (double)x.rows * x.cols;
-            if (single(x)) {
-                if (x.s1 == x.s0) G.src[k] = {-1, 0.0};
-                else G.src[k] = {P.wapply.srcs[x.s0].off, P.wapply.srcs[x.s0].coef};
-                continue;
+    parallel_for(
+        (int)segs.size(),
+        [&](int i) {
+            const Seg &sg = segs[i];
+            const int rsz = s.rsize(sg.ar);
+            int64_t a = nst[i], b = nsr[i], dst = P.n_t + el[i];
+            for (int64_t k = first[i]; k < first[i + 1]; ++k) {
+                const Strip &x = st[k];
+                if (x.s1 > x.s0) read[i] += (double)x.rows * x.cols;
+                if (single(x)) {
+                    if (x.s1 == x.s0) G.src[k] = {-1, 0.0};
+                    else G.src[k] = {P.wapply.srcs[x.s0].off, P.wapply.srcs[x.s0].coef};
+                    continue;
+                }
+                G.src[k] = {dst, 1.0};
+                out.strips[a++] = {dst, x.rows, x.cols, x.rows, (int)b, (int)b + x.s1 - x.s0};
+                for (int q = x.s0; q < x.s1; ++q) out.srcs[b++] = P.wapply.srcs[q];
+                dst += (int64_t)x.rows * x.cols;
             }
-            G.src[k] = {dst, 1.0};
-            out.strips[a++] = {dst, x.rows, x.cols, x.rows, (int)b, (int)b + x.s1 - x.s0};
-            for (int q = x.s0; q < x.s1; ++q) out.srcs[b++] = P.wapply.srcs[q];
-            dst += (int64_t)x.rows * x.cols;
-        }
-        for (int k = 0; k < rsz; k += 4)
-            G.quad[q0[sg.al] + (sg.koff + k) / 4] = {(int)first[i], 8 * k + std::min(4, rsz - k)};
-    });
+            for (int k = 0; k < rsz; k += 4)
+                G.quad[q0[sg.al] + (sg.koff + k) / 4] = {(int)first[i], 8 * k + std::min(4, rsz - k)};
+        },
+        grain);
     for (double r : read) G.elements += r;
     for (auto &g : P.g2.groups) {  // c is the al block's offset in sigma
         for (auto &xb : s.X.blk)
