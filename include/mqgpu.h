@@ -150,8 +150,9 @@ const char *mq_last_error(const mq_ctx *ctx);
  * repeat at few positions are summed on the left boundary first, 2 every
  * column is summed that way (testing aid).  Under mode 1 a column is summed
  * that way when its entries number at least MQ_OPT_FUSE_MIN (1..4095, default
- * 64) and at least MQ_OPT_FUSE_RATIO (1..255, default 4) times its distinct
- * positions or 2 * MQ_OPT_FUSE_RATIO times its output states.  MQ_OPT_KCHUNK: target K chunk of split-K GEMM
+ * 64) and either at least MQ_OPT_FUSE_RATIO (1..255, default 4) times its
+ * distinct positions, or at least 2 * MQ_OPT_FUSE_RATIO times its output states
+ * and MQ_OPT_FUSE_RATIO / 2 times its positions.  MQ_OPT_KCHUNK: target K chunk of split-K GEMM
  * groups (256..65536, a multiple of 16, default 2048).  Results agree to
  * round-off.  MQ_OPT_GRAPH (0 default / 1): the Davidson drivers run their
  * sigma vectors through mq_sigma_graph's captured graph (same results).
