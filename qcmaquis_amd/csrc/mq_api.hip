@@ -1170,8 +1170,11 @@ struct JD {
     }
 };
 
-// cyclic Jacobi eigen-decomposition of a small symmetric matrix (column-major)
-void sym_eig(int n, std::vector<double> A, std::vector<double> &w, std::vector<double> &V) {
+// cyclic Jacobi eigen-decomposition of a small symmetric matrix (column-major).  On a cache
+// line of its own: where its inner loops fall otherwise follows the code before it, and
+// decides up to a quarter of its time (130 vectors, on the GPU's host: 11.5 ms at 0 or 48
+// bytes into a line, 14.5 ms at 16).
+__attribute__((aligned(64))) void sym_eig(int n, std::vector<double> A, std::vector<double> &w, std::vector<double> &V) {
     V.assign((size_t)n * n, 0.0);
     for (int i = 0; i < n; ++i) V[(size_t)i * n + i] = 1.0;
     for (int sweep = 0; sweep < 100; ++sweep) {
