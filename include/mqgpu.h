@@ -409,6 +409,11 @@ int mq_gemm_f32(mq_ctx *ctx, int transA, int transB, int M, int N, int K,
                 const float *A, int lda, const float *B, int ldb,
                 float *C, int ldc, int kchunk, int tm, int tn, int bf16x3);
 
+/* t (n elements) orthonormalised in place against the m <= 1000 orthonormal vectors V (one
+ * after another), as a Jacobi-Davidson iteration does (jacobi.h:384-393): Gram-Schmidt,
+ * repeated when the norm drops below a quarter of its value, and normalisation. */
+int mq_orthonormalise(mq_ctx *ctx, const double *V, int64_t n, int m, double *t);
+
 /* -- host-side plan introspection (no GPU needed) ------------------------ */
 /* Builds the same task lists the device plans execute, on the host only, so
  * that schedules, FLOP counts and workspace sizes can be inspected (and the

@@ -1243,6 +1243,69 @@ struct Stall {
     }
 };
 
+// Orthonormalisation on the device alone: t against the first m vectors of V (orthonormal,
+// one after another) and the n_ortho vectors O, whose inverse squared norms are ow.  p0 .. p3
+// hold partials (rows of nblk: t.t, then one per vector).
+struct Orth {
+    const double *V;
+    int64_t n;
+    const double *O, *ow;
+    int n_ortho;
+    double *p0, *p1, *p2, *p3;
+    int nblk;
+    hipStream_t s;
+    // the dots of t with itself and the first m vectors of V into p0
+    void dots(int m, double *t) const {
+        check(launch_orth(ORTH_DOTS, V, n, m, t, nullptr, nullptr, nullptr, nullptr, nullptr, true, nblk, p0, s), "norm");
+    }
+    // SingleSiteVS::project (ietl_lanczos_solver.h:90-95); leaves the dots of t in p3
+    void project(double *t) const {
+        if (n_ortho == 0) return;
+        check(launch_orth(ORTH_DOTS, O, n, n_ortho, t, nullptr, nullptr, nullptr, nullptr, nullptr, true, nblk, p2, s),
+              "project");
+        check(launch_orth(ORTH_UPDATE, O, n, n_ortho, t, nullptr, nullptr, ow, p2, nullptr, true, nblk, p3, s),
+              "project");
+    }
+    // t with its dots in p0 (jacobi.h:384-393: Gram-Schmidt, repeated when the norm drops
+    // below a quarter of its value)
+    void run(int m, double *t) const {
+        if (m > 0) {
+            check(launch_orth(ORTH_UPDATE, V, n, m, t, nullptr, nullptr, nullptr, p0, nullptr, true, nblk, p1, s),
+                  "orthogonalise");
+            check(launch_orth(ORTH_UPDATE, V, n, m, t, nullptr, nullptr, nullptr, p1, p0, true, nblk, p2, s),
+                  "orthogonalise");
+        }
+        project(t);
+        if (n_ortho > 0)
+            check(launch_normalise(t, n, nblk, nullptr, p3, nullptr, s), "normalise");
+        else if (m > 0)
+            check(launch_normalise(t, n, nblk, p0, p1, p2, s), "normalise");
+        else
+            check(launch_normalise(t, n, nblk, nullptr, p0, nullptr, s), "normalise");
+    }
+};
+
+extern "C" int mq_orthonormalise(mq_ctx *ctx, const double *V, int64_t n, int m, double *t) {
+    if (!ctx) return MQ_ERR_ARG;
+    if (!t || n < 1 || m < 0 || m > 1000 || (m > 0 && !V)) {
+        ctx->err = "mq_orthonormalise: needs n >= 1 and m in 0..1000";
+        return MQ_ERR_ARG;
+    }
+    try {
+        const int nblk = (int)std::max<int64_t>(1, std::min<int64_t>(kJdBlocks, (n + 255) / 256));
+        const size_t part = (size_t)(m + 1) * nblk;
+        DevArray<double> p;
+        p.alloc(3 * part);
+        const Orth orth{V, n, nullptr, nullptr, 0, p.p, p.p + part, p.p + 2 * part, nullptr, nblk, ctx->stream};
+        orth.dots(m, t);
+        orth.run(m, t);
+        check(hipStreamSynchronize(ctx->stream), "orthonormalise");
+        return MQ_OK;
+    } catch (std::exception &e) {
+        return fail(ctx, e, MQ_ERR_HIP);
+    }
+}
+
 extern "C" int mq_jacobi_davidson(mq_plan *plan, const double *L, const double *R, const double *x0, double *u_out,
                                   double *theta_out, int max_iter, double tol, int prec, const double *const *ortho,
                                   int n_ortho, int *iterations) {
@@ -1294,41 +1357,12 @@ extern "C" int mq_jacobi_davidson(mq_plan *plan, const double *L, const double *
             check(hipMemcpyAsync(ow, oo.data(), sizeof(double) * n_ortho, hipMemcpyHostToDevice, jd.s), "ortho norms");
             jd.sync();  // oo goes out of scope
         }
-        // SingleSiteVS::project (ietl_lanczos_solver.h:90-95); leaves the dots of t in p3
-        auto project = [&](double *t) {
-            if (n_ortho == 0) return;
-            check(launch_orth(ORTH_DOTS, O, n, n_ortho, t, nullptr, nullptr, nullptr, nullptr, nullptr, true, jd.nblk,
-                              p2, jd.s),
-                  "project");
-            check(launch_orth(ORTH_UPDATE, O, n, n_ortho, t, nullptr, nullptr, ow, p2, nullptr, true, jd.nblk, p3,
-                              jd.s),
-                  "project");
-        };
-        // orthonormalise t = V(m), its dots in p0 (jacobi.h:384-393: Gram-Schmidt, repeated
-        // when the norm drops below a quarter of its value), on the device alone
-        auto orthonormalise = [&](int m) {
-            double *t = V(m);
-            if (m > 0) {
-                check(launch_orth(ORTH_UPDATE, V(0), n, m, t, nullptr, nullptr, nullptr, p0, nullptr, true, jd.nblk,
-                                  p1, jd.s),
-                      "orthogonalise");
-                check(launch_orth(ORTH_UPDATE, V(0), n, m, t, nullptr, nullptr, nullptr, p1, p0, true, jd.nblk, p2,
-                                  jd.s),
-                      "orthogonalise");
-            }
-            project(t);
-            if (n_ortho > 0)
-                check(launch_normalise(t, n, jd.nblk, nullptr, p3, nullptr, jd.s), "normalise");
-            else if (m > 0)
-                check(launch_normalise(t, n, jd.nblk, p0, p1, p2, jd.s), "normalise");
-            else
-                check(launch_normalise(t, n, jd.nblk, nullptr, p0, nullptr, jd.s), "normalise");
-        };
+        const Orth orth{V(0), n, O, ow, n_ortho, p0, p1, p2, p3, jd.nblk, jd.s};
+        auto project = [&](double *t) { orth.project(t); };
+        auto orthonormalise = [&](int m) { orth.run(m, V(m)); };
         check(hipMemcpyAsync(V(0), x0, sizeof(double) * n, hipMemcpyDeviceToDevice, jd.s), "x0");
         project(V(0));
-        check(launch_orth(ORTH_DOTS, V(0), n, 0, V(0), nullptr, nullptr, nullptr, nullptr, nullptr, true, jd.nblk, p0,
-                          jd.s),
-              "norm");
+        orth.dots(0, V(0));
         orthonormalise(0);
         std::vector<double> M((size_t)max_iter * max_iter, 0.0);
         int it = 0;

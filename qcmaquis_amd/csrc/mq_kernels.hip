@@ -844,21 +844,49 @@ __device__ inline void two_sum(double &hi, double &lo, double x) {
     lo += (hi - (s - z)) + (x - z);
     hi = s;
 }
-// sum of one row of partials by a wave, in twice the working precision (as the host's
-// long double sums were at least)
-__device__ inline double row_sum(const double *__restrict__ row, int nblk, int lane) {
-    double hi = 0.0, lo = 0.0;
-    for (int b = lane; b < nblk; b += 64) two_sum(hi, lo, row[b]);
-    for (int o = 32; o > 0; o >>= 1) {
-        const double h2 = __shfl_xor(hi, o, 64), l2 = __shfl_xor(lo, o, 64);
-        two_sum(hi, lo, h2);
-        lo += l2;
+// sums of R rows of partials by a wave, in twice the working precision (as the host's long
+// double sums were at least).  A row's sum is a chain of loads and shuffles of about 2 us,
+// so several rows go side by side.
+template <int R>
+__device__ inline void row_sums(const double *const (&row)[R], int nblk, int lane, double (&sum)[R]) {
+    double hi[R], lo[R];
+#pragma unroll
+    for (int k = 0; k < R; ++k) hi[k] = lo[k] = 0.0;
+    for (int b0 = 0; b0 < nblk; b0 += 256) {
+        double x[R][4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int b = b0 + lane + 64 * q;
+#pragma unroll
+            for (int k = 0; k < R; ++k) {
+                x[k][q] = row[k][min(b, nblk - 1)];
+                if (b >= nblk) x[k][q] = 0.0;
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int k = 0; k < R; ++k) two_sum(hi[k], lo[k], x[k][q]);
     }
-    return __shfl(hi + lo, 0, 64);  // one lane's rounding for all
+    for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            const double h2 = __shfl_xor(hi[k], o, 64), l2 = __shfl_xor(lo[k], o, 64);
+            two_sum(hi[k], lo[k], h2);
+            lo[k] += l2;
+        }
+#pragma unroll
+    for (int k = 0; k < R; ++k) sum[k] = __shfl(hi[k] + lo[k], 0, 64);  // one lane's rounding for all
 }
-// block sums of up to 4 per-thread values
+__device__ inline double row_sum(const double *row, int nblk, int lane) {
+    double s[1];
+    const double *const r[1] = {row};
+    row_sums<1>(r, nblk, lane, s);
+    return s[0];
+}
+// block sums of N per-thread values: thread k < N returns the k-th (red: N per wave)
 template <int N>
-__device__ inline void block_sums(double (&v)[N], double *red) {
+__device__ inline double block_sums(double (&v)[N], double *red) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
     for (int k = 0; k < N; ++k)
@@ -868,56 +896,90 @@ __device__ inline void block_sums(double (&v)[N], double *red) {
 #pragma unroll
         for (int k = 0; k < N; ++k) red[wave * N + k] = v[k];
     __syncthreads();
-#pragma unroll
-    for (int k = 0; k < N; ++k) v[k] = (red[k] + red[N + k]) + (red[2 * N + k] + red[3 * N + k]);
+    double s = 0.0;
+    if ((int)threadIdx.x < N)
+        for (int w = 0; w < (int)blockDim.x >> 6; ++w) s += red[w * N + threadIdx.x];
+    return s;
 }
 
 // MODE 0: dots of t.  MODE 1: t = f u - r first, f = (r.u)/(u.u) from pin rows 1, 2.
 // MODE 2: t -= sum_i w_i (V_i.t) V_i first, the products from pin (w null: all 1); with
 // ptau, only when |t| (pin row 0) fell below a quarter of ptau's row 0, the
 // refinement test of jacobi.h:384-393.  Block b owns elements [b * chunk, (b+1) * chunk).
+// Eight basis vectors are loaded before they are used, a wave sums four rows of partials side
+// by side, and a block has kOrthThreads threads when its chunk fills 256: a long basis of
+// long vectors is read at the rate that the loads in flight allow.  An iteration's time
+// beside the sigma, mean of 60 iterations at n = 340,000 (the Rayleigh eigenproblem, 320 us
+// on the host, among it): 525 us with host-driven steps, 612 us with four vectors, each under
+// its own condition, 256 threads and one row at a time, 453 us so; mean of 30: 162, 150, 81.
+constexpr int kOrthThreads = 512, kOrthVecs = 8;
 template <int MODE>
-__global__ void __launch_bounds__(256) k_orth(const double *__restrict__ V, int64_t n, int64_t chunk, int m,
-                                              double *t, const double *u, const double *r,
-                                              const double *__restrict__ w, const double *__restrict__ pin,
-                                              const double *__restrict__ ptau, int self,
-                                              double *__restrict__ pout) {
+__global__ void __launch_bounds__(kOrthThreads) k_orth(const double *__restrict__ V, int64_t n, int64_t chunk, int m,
+                                                       double *t, const double *u, const double *r,
+                                                       const double *__restrict__ w, const double *__restrict__ pin,
+                                                       const double *__restrict__ ptau, int self,
+                                                       double *__restrict__ pout) {
     extern __shared__ double coef[];  // m
-    __shared__ double red[16];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nblk = gridDim.x;
+    __shared__ double red[(kOrthThreads / 64) * (kOrthVecs + 1)];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nblk = gridDim.x, nt = blockDim.x;
     const int64_t lo = blockIdx.x * chunk, hi = min(n, lo + chunk);
     if (MODE == 1) {
-        const double f = row_sum(pin + nblk, nblk, lane) / row_sum(pin + 2 * nblk, nblk, lane);
-        for (int64_t e = lo + threadIdx.x; e < hi; e += 256) t[e] = fma(f, u[e], -r[e]);
+        const double *const row[2] = {pin + nblk, pin + 2 * nblk};
+        double d[2];
+        row_sums<2>(row, nblk, lane, d);
+        const double f = d[0] / d[1];
+        for (int64_t e = lo + threadIdx.x; e < hi; e += nt) t[e] = fma(f, u[e], -r[e]);
     }
     if (MODE == 2) {
         if (ptau && sqrt(row_sum(pin, nblk, lane)) >= 0.25 * sqrt(row_sum(ptau, nblk, lane))) return;
-        for (int i = wave; i < m; i += 4) {
-            const double d = row_sum(pin + (int64_t)(i + 1) * nblk, nblk, lane);
-            if (lane == 0) coef[i] = w ? d * w[i] : d;
+        for (int i = 4 * wave; i < m; i += nt >> 4) {  // four rows per wave
+            const double *row[4];
+            double d[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) row[k] = pin + (int64_t)(min(i + k, m - 1) + 1) * nblk;
+            row_sums<4>({row[0], row[1], row[2], row[3]}, nblk, lane, d);
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                if (lane == 0 && i + k < m) coef[i + k] = w ? d[k] * w[i + k] : d[k];
         }
         __syncthreads();
-        for (int64_t e = lo + threadIdx.x; e < hi; e += 256) {
+        for (int64_t e = lo + threadIdx.x; e < hi; e += nt) {
             double a = t[e];
-            for (int i = 0; i < m; ++i) a = fma(-coef[i], V[i * n + e], a);
+            int i = 0;
+            for (; i + kOrthVecs <= m; i += kOrthVecs) {
+                double x[kOrthVecs];
+#pragma unroll
+                for (int q = 0; q < kOrthVecs; ++q) x[q] = V[(i + q) * n + e];
+#pragma unroll
+                for (int q = 0; q < kOrthVecs; ++q) a = fma(-coef[i + q], x[q], a);
+            }
+            for (; i < m; ++i) a = fma(-coef[i], V[i * n + e], a);
             t[e] = a;
         }
     }
     // each thread reads back only elements it wrote itself
-    for (int p = self ? -1 : 0; p < m; p += 4) {
-        double acc[4] = {0, 0, 0, 0};
-        const int k = min(4, m - p);
-        for (int64_t e = lo + threadIdx.x; e < hi; e += 256) {
-            const double x = t[e];
+    for (int p = 0; p < max(m, self); p += kOrthVecs) {
+        double acc[kOrthVecs + 1];
+        const double *v[kOrthVecs];
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
-                if (q < k) acc[q] = fma(p + q < 0 ? x : V[(p + q) * n + e], x, acc[q]);
+        for (int q = 0; q < kOrthVecs; ++q) {
+            acc[q] = 0.0;
+            v[q] = m > 0 ? V + (int64_t)min(p + q, m - 1) * n : t;  // past the end: read, not used
         }
-        block_sums<4>(acc, red);
-        if (threadIdx.x < 4 && (int)threadIdx.x < k) {
-            const double s = threadIdx.x == 0 ? acc[0] : threadIdx.x == 1 ? acc[1] : threadIdx.x == 2 ? acc[2] : acc[3];
-            pout[(int64_t)(p + (int)threadIdx.x + (self ? 1 : 0)) * nblk + blockIdx.x] = s;
+        acc[kOrthVecs] = 0.0;
+        for (int64_t e = lo + threadIdx.x; e < hi; e += nt) {
+            const double x = t[e];
+            double y[kOrthVecs];
+#pragma unroll
+            for (int q = 0; q < kOrthVecs; ++q) y[q] = v[q][e];
+#pragma unroll
+            for (int q = 0; q < kOrthVecs; ++q) acc[q] = fma(y[q], x, acc[q]);
+            acc[kOrthVecs] = fma(x, x, acc[kOrthVecs]);
         }
+        const double s = block_sums<kOrthVecs + 1>(acc, red);
+        const int k = threadIdx.x;
+        if (k < min(kOrthVecs, m - p)) pout[(int64_t)(p + k + self) * nblk + blockIdx.x] = s;
+        if (k == kOrthVecs && self && p == 0) pout[blockIdx.x] = s;
     }
 }
 
@@ -936,16 +998,29 @@ __global__ void __launch_bounds__(256) k_normalise(double *t, int64_t n, int nbl
 // u = sum c V, r = sum c VA - theta u, and the partials of r.r, r.u, u.u (to device and
 // pinned host memory): one pass over the two bases.  Bases beyond kCombMax vectors
 // take several launches: `first` starts the sums, `last` forms r.
-__global__ void __launch_bounds__(256) k_ritz(const RitzArgs c, int nv, const double *__restrict__ V,
-                                              const double *__restrict__ VA, int64_t n, double theta, int first,
-                                              int last, double *u, double *r, double *__restrict__ pdev,
-                                              double *__restrict__ phost) {
-    __shared__ double red[12];
+__global__ void __launch_bounds__(kOrthThreads) k_ritz(const RitzArgs c, int nv, const double *__restrict__ V,
+                                                       const double *__restrict__ VA, int64_t n, double theta,
+                                                       int first, int last, double *u, double *r,
+                                                       double *__restrict__ pdev, double *__restrict__ phost) {
+    __shared__ double red[3 * kOrthThreads / 64];
     double acc[3] = {0, 0, 0};
     for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < n; e += (int64_t)gridDim.x * blockDim.x) {
         double a = first ? 0.0 : u[e], b = first ? 0.0 : r[e];
-#pragma unroll 4
-        for (int j = 0; j < nv; ++j) {
+        int j = 0;
+        for (; j + 4 <= nv; j += 4) {
+            double x[4], y[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                x[q] = V[(j + q) * n + e];
+                y[q] = VA[(j + q) * n + e];
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                a = fma(c.c[j + q], x[q], a);
+                b = fma(c.c[j + q], y[q], b);
+            }
+        }
+        for (; j < nv; ++j) {
             a = fma(c.c[j], V[j * n + e], a);
             b = fma(c.c[j], VA[j * n + e], b);
         }
@@ -957,12 +1032,11 @@ __global__ void __launch_bounds__(256) k_ritz(const RitzArgs c, int nv, const do
         acc[2] = fma(a, a, acc[2]);
     }
     if (!last) return;
-    block_sums<3>(acc, red);
-    if (threadIdx.x == 0)
-        for (int k = 0; k < 3; ++k) {
-            pdev[k * gridDim.x + blockIdx.x] = acc[k];
-            phost[k * gridDim.x + blockIdx.x] = acc[k];
-        }
+    const double x = block_sums<3>(acc, red);
+    if (threadIdx.x < 3) {
+        pdev[threadIdx.x * gridDim.x + blockIdx.x] = x;
+        phost[threadIdx.x * gridDim.x + blockIdx.x] = x;
+    }
 }
 
 // ------------------------------------------------------------------ launchers
@@ -1118,7 +1192,7 @@ hipError_t launch_orth(OrthMode mode, const double *V, int64_t n, int m, double 
                        const double *w, const double *pin, const double *ptau, bool self, int nblocks, double *pout,
                        hipStream_t s) {
     const int64_t chunk = (n + nblocks - 1) / nblocks;
-    const dim3 g(nblocks), b(256);
+    const dim3 g(nblocks), b(chunk > 256 ? kOrthThreads : 256);
     const size_t lds = sizeof(double) * std::max(1, m);
     if (mode == ORTH_DOTS)
         hipLaunchKernelGGL((k_orth<0>), g, b, lds, s, V, n, chunk, m, t, u, r, w, pin, ptau, self, pout);
@@ -1137,7 +1211,7 @@ hipError_t launch_normalise(double *t, int64_t n, int nblocks, const double *p0,
 hipError_t launch_ritz(const RitzArgs &c, int nv, const double *V, const double *VA, int64_t n, double theta,
                        bool first, bool last, double *u, double *r, int nblocks, double *pdev, double *phost,
                        hipStream_t s) {
-    hipLaunchKernelGGL(k_ritz, dim3(nblocks), dim3(256), 0, s, c, nv, V, VA, n, theta, first, last, u, r, pdev, phost);
+    hipLaunchKernelGGL(k_ritz, dim3(nblocks), dim3(n > (int64_t)256 * nblocks ? kOrthThreads : 256), 0, s, c, nv, V, VA, n, theta, first, last, u, r, pdev, phost);
     return hipGetLastError();
 }
 __global__ void __launch_bounds__(256) k_diag_scale(const double *x, const double *u, double f,

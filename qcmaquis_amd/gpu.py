@@ -65,6 +65,7 @@ def lib():
                                   C.c_int, C.c_int]
         L.mq_gemm_f32.argtypes = [vp, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, vp, C.c_int, vp, C.c_int, vp,
                                   C.c_int, C.c_int, C.c_int, C.c_int, C.c_int]
+        L.mq_orthonormalise.argtypes = [vp, vp, C.c_int64, C.c_int, vp]
         L.mq_step_out_desc.argtypes = [vp, C.POINTER(mq_boundary_desc)]
         L.mq_boundary_step.argtypes = [vp, vp, vp, vp]
         L.mq_jacobi_davidson.argtypes = [vp, vp, vp, vp, vp, f64p, C.c_int, C.c_double, C.c_int,
@@ -302,6 +303,17 @@ class GpuEngine:
         self.check(lib().mq_gemm_f32(self.ctx, int(transA), int(transB), M, N, K, _ptr(A), max(lda, 1), _ptr(B),
                                      max(ldb, 1), _ptr(Cm), max(M, 1), kchunk, tm, tn, int(bf16x3)), "mq_gemm_f32")
         return Cm.t()
+
+    def orthonormalise(self, V, t):
+        """t orthonormalised in place against the orthonormal rows of V (FP64 device tensors)."""
+        if V.shape[1:] != t.shape or not (V.is_contiguous() and t.is_contiguous()):
+            raise ValueError("orthonormalise: V must be (m, n) and t (n,), both contiguous")
+        for x in (V, t):
+            if x.dtype != self.torch.float64 or x.device != self.device:
+                raise ValueError("orthonormalise: FP64 tensors on the engine's device")
+        self.torch.cuda.synchronize()
+        self.check(lib().mq_orthonormalise(self.ctx, _ptr(V), t.numel(), V.shape[0], _ptr(t)), "mq_orthonormalise")
+        return t
 
     def seed_boundary(self, charge):
         return GpuBoundary(BoundaryLayout.seed(charge), self.to_dev(np.ones(1)))
