@@ -2129,13 +2129,16 @@ int mq_host_plan_create(const mq_site_desc *desc, int kind, mq_host_plan **out) 
     try {
         std::unique_ptr<mq_host_plan> h(new mq_host_plan());
         const int tm = 0, tn = 0, kc = 2048;
-        const int fm = (kind >> 8) & 3, fr = (kind >> 10) & 255, fmin = (kind >> 18) & 4095, k = kind & 15;
+        const int fm = (kind >> 8) & 3, fr = (kind >> 10) & 255, fmin = (kind >> 18) & 4095;
+        const bool gather = (kind & MQ_HOST_GATHER) != 0;
+        const int k = kind & 255 & ~MQ_HOST_GATHER;
+        if (gather && k != PLAN_SIGMA) return MQ_ERR_ARG;
         FuseRule fuse;
         if (fm) fuse.mode = fm - 1;
         if (fr) fuse.ratio = fr;
         if (fmin) fuse.min_entries = fmin;
         const int sched = (kind >> 30) & 1;
-        if (k == PLAN_SIGMA) h->hp = build_sigma_plan(*desc, tm, tn, kc, fuse, true, sched, (kind & MQ_HOST_GATHER) != 0);
+        if (k == PLAN_SIGMA) h->hp = build_sigma_plan(*desc, tm, tn, kc, fuse, true, sched, gather);
         else if (k == PLAN_LSTEP) h->hp = build_lstep_plan(*desc, tm, tn, kc, fuse);
         else if (k == PLAN_RSTEP) h->hp = build_rstep_plan(*desc, tm, tn, kc);
         else if (k == PLAN_DIAG) h->hp = build_diag_plan(*desc, tm, tn, kc);
