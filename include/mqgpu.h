@@ -152,10 +152,12 @@ const char *mq_last_error(const mq_ctx *ctx);
  * that way when its entries number at least MQ_OPT_FUSE_MIN (1..4095, default
  * 64) and either at least MQ_OPT_FUSE_RATIO (1..255, default 4) times its
  * distinct positions, or at least 2 * MQ_OPT_FUSE_RATIO times its output states
- * and MQ_OPT_FUSE_RATIO / 2 times its positions.  MQ_OPT_KCHUNK: target K chunk of split-K GEMM
- * groups (256..65536, a multiple of 16, default 2048).  Results agree to
- * round-off.  MQ_OPT_GRAPH (0 default / 1): the Davidson drivers run their
- * sigma vectors through mq_sigma_graph's captured graph (same results).
+ * and MQ_OPT_FUSE_RATIO / 2 times its positions.  MQ_OPT_KCHUNK: the largest K
+ * chunk of a plan's split-K GEMM groups (256..65536, a multiple of 16, default
+ * 2048); a launch of fewer than 1024 tiles gets smaller ones, as many as fill it,
+ * down to 128.  Results agree to round-off.  MQ_OPT_GRAPH (0 default / 1): the
+ * Davidson drivers run their sigma vectors through mq_sigma_graph's captured
+ * graph (same results).
  * MQ_OPT_TILE_M: row tile of every GEMM group, 64 or 128, or 0 (default:
  * 128 rows unless the group's M fits 64).  MQ_OPT_REF_FLOPS (1 default / 0):
  * count the reference schedule's FLOPs for mq_plan_flops; with 0 sigma and

@@ -5,7 +5,8 @@ results do not (they agree to round-off):
   - the fused-column rule: which MPO columns are summed on the left boundary
     first (mode 0 none, 1 by an entries/positions ratio and a minimum entry
     count, 2 all), trading W-application traffic for GEMM flops;
-  - the split-K chunk of the output GEMM groups;
+  - the largest split-K chunk of the GEMM groups (a launch that does not fill the GPU
+    gets a smaller one, and then the same plan for all of them);
   - the GEMM row tile (0: 128 rows unless a group fits 64; or 64 for every group,
     twice the tiles with half the accumulators each);
   - the GEMM column tile (0: per group the width that wastes the fewest padded
@@ -16,7 +17,7 @@ library stream, and keeps the fastest.  Results are cached per site shape
 (the MPO bond dimensions and the boundary and vector sizes), so a sweep tunes
 each distinct problem once.
 """
-from dataclasses import dataclass, asdict
+from dataclasses import asdict, dataclass, replace
 
 import numpy as np
 
@@ -67,9 +68,11 @@ def site_key(symm, psi, L, R, W):
     return (symm, W.row_dim, W.col_dim, psi.to_flat().size, L.layout.total, R.layout.total)
 
 
-def time_schedule(engine, symm, psi, L, R, W, sched, x, prec, reps=5, warmup=2):
+def time_schedule(engine, symm, psi, L, R, W, sched, x, prec, reps=5, warmup=2, known=None):
     """Median stage-summed sigma time (ms) of one schedule, and the plan's
-    executed FLOPs and workspace bytes."""
+    executed FLOPs and workspace bytes.  known: such a row of a schedule that differs in
+    the K chunk alone, returned as it is when the plans are the same (a chunk changes the
+    number of partial tiles, and the workspace with it, unless it changes no group's split)."""
     prev = getattr(engine, "schedule", DEFAULT)
     engine.set_schedule(sched)
     try:
@@ -77,6 +80,8 @@ def time_schedule(engine, symm, psi, L, R, W, sched, x, prec, reps=5, warmup=2):
     finally:
         engine.set_schedule(prev)
     try:
+        if known and known[1:] == (sp.exec_flops, sp.workspace_bytes):
+            return known
         y = engine.torch.empty_like(x)
         for _ in range(warmup):
             sp.apply(x, y, prec=prec)
@@ -102,7 +107,8 @@ def tune(engine, symm, psi, L, R, W, prec=MQ_PREC_FP64, cands=None, reps=5, log=
     x = engine.to_dev(np.random.default_rng(7).standard_normal(psi.to_flat().size))
     table = []
     for s in (cands or candidates()):
-        ms, ex, ws = time_schedule(engine, symm, psi, L, R, W, s, x, prec, reps)
+        known = [r[1:] for r in table if r[0] == DEFAULT and replace(s, kchunk=DEFAULT.kchunk) == DEFAULT]
+        ms, ex, ws = time_schedule(engine, symm, psi, L, R, W, s, x, prec, reps, known=known[0] if known else None)
         table.append((s, ms, ex, ws))
         if log:
             log(f"  schedule {s.label()}: {ms:.3f} ms, executed {ex / 1e9:.1f} GF, workspace {ws / 1e9:.2f} GB")
