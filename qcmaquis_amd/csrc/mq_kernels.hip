@@ -40,7 +40,8 @@ __global__ void __launch_bounds__(256) k_to_f32(const double *__restrict__ src, 
 // ------------------------------------------------------------------ W application
 // dst strip = sum_s coef_s * src_s, summed in task order (deterministic, no
 // atomics).  Element e of a strip is (i, j) = (e mod rows, e / rows), the quotient taken
-// from a float reciprocal and corrected (exact for strips below 2^24 elements).
+// from a float reciprocal and corrected by one (exact below kStripCols columns: the float
+// quotient is off by less than 4 / 2^24 of itself; make_packs refuses wider strips).
 constexpr int WU = 4;
 
 // One pass over a large strip: each thread owns WS = 8 elements, so that a wave has

@@ -1361,7 +1361,8 @@ void make_packs(StripList &sl) {
     int i = 0;
     while (i < n) {
         int64_t el = elems(i);
-        if (el >= INT32_MAX - kPassElems) throw std::runtime_error("strip too large");
+        if (sl.strips[i].cols >= kStripCols || el + 2ll * sl.strips[i].rows > INT32_MAX - kPassElems)
+            throw std::runtime_error("strip too large");
         int j = i + 1;
         if (el > kPackElems) {
             for (int e = 0; e < el; e += kPassElems) sl.packs.push_back({i, 1, e});

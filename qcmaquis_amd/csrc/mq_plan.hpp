@@ -128,6 +128,8 @@ struct GemmList {
 // elements of one strip, from e0 on.
 constexpr int kPackStrips = 64, kPackElems = 1024, kPassElems = 2048, kChainSrcs = 8;
 constexpr int kPackSmall = -1, kPackWaves = -2;
+// a strip has fewer columns than this, and its elements and two columns more fit an int
+constexpr int kStripCols = 1 << 22;
 struct Pack {
     int first, n;  // strips [first, first + n)
     int e0;        // kPackSmall, kPackWaves, or the first element of the one strip's pass
