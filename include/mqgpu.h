@@ -149,10 +149,9 @@ const char *mq_last_error(const mq_ctx *ctx);
  * are evaluated -- 0 term by term, 1 (default) columns whose operator entries
  * repeat at few positions are summed on the left boundary first, 2 every
  * column is summed that way (testing aid).  Under mode 1 a column is summed
- * that way when its entries number at least MQ_OPT_FUSE_MIN (1..4095, default
- * 64) and either at least MQ_OPT_FUSE_RATIO (1..255, default 4) times its
- * distinct positions, or at least 2 * MQ_OPT_FUSE_RATIO times its output states
- * and MQ_OPT_FUSE_RATIO / 2 times its positions.  MQ_OPT_KCHUNK: the largest K
+ * that way when its entries number at least MQ_OPT_FUSE_RATIO (1..255, default
+ * 4) times its distinct positions and at least MQ_OPT_FUSE_MIN (1..4095,
+ * default 64).  MQ_OPT_KCHUNK: the largest K
  * chunk of a plan's split-K GEMM groups (256..65536, a multiple of 16, default
  * 2048); a launch of fewer than 1024 tiles gets smaller ones, as many as fill it,
  * down to 128.  Results agree to round-off.  MQ_OPT_GRAPH (0 default / 1): the

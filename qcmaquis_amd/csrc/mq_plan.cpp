@@ -459,26 +459,16 @@ struct ColProg {
     std::vector<char> direct, member;     // [b1] row has direct terms / feeds a fused column
 };
 
-// Columns are fused by fuse.mode: 0 none, 2 every non-empty one (used by tests to exercise
-// fused columns on small systems), 1 those of at least fuse.min_entries entries that number
-//  - fuse.ratio times their distinct positions, or
-//  - 2 * fuse.ratio times their output states and fuse.ratio / 2 times their positions.
-// The second rule is about the chain of sources that every element of the column's C rows
-// sums in the W application, which bounds it in small problems.  A fused column costs
-// host time per position and left block, so the entries have to merge: without the
-// fuse.ratio / 2 the rule also takes columns near a chain's end whose sums have 1.2 entries
-// each.  Measured, us (plan build, sigma, and plan + binding + ten Jacobi-Davidson
-// iterations; one MI355X, FP64 unless said otherwise):
-//                            first rule only      no fuse.ratio / 2      both rules
-//   SU2U1 L=8  m=30  site 1  1294   78   2136     2608   69   3460     1393   69   2207
-//   SU2U1 L=12 m=100 site 2  3195   78   4065     5934   69   6734     4891   70   5761
-//   SU2U1 L=16 m=201 site 5 13804  136  15359    15929  123  17355    15674  123  17105
-//     the same, BF16x3               122                   96                   98
-//   TwoU1 L=8  m=40  site 3  5350   73   6186     6760   78   7651     6310   78   7195
-//   TwoU1 L=12 m=200 site 5 19780  193  21939    22117  189  24280    20261  189  22402
-//     the same, BF16x3               157                  139                  137
-//   SU2U1 L=24 m=512 centre 75779 3532 118333    74496 3532 117037    75561 3527 118115
-//   TwoU1 L=24 m=512 centre 57891 2557  88854    58117 2569  89087    58212 2568  89217
+// fuse.mode: 0 never, 1 when a column's entries are at least fuse.ratio times its
+// distinct positions and number at least fuse.min_entries, 2 every non-empty
+// column (used by tests to exercise fused columns on small systems).
+// Fusing also by the entries per output state (the chain of sources that each element of
+// the column's C rows sums in the W application) was measured and taken back.  It made the
+// sigma of small problems faster (L=16 m=201 BF16x3 122 -> 96 us, L=8 m=30 site 2 74 -> 65),
+// but such columns' entries hardly merge: a plan took up to twice as long (L=8 m=30 site 1
+// 1.3 -> 2.6 ms), which a hundred iterations do not give back, and BF16x3 lost precision,
+// the sums being split once into bf16 parts where the terms' errors had averaged (against
+// 64 bits 1.9e-5 -> 2.5e-5 at L=8 m=30 site 1, 2.3e-5 -> 3.4e-5 at L=8 m=74 site 3).
 ColProg column_program(const Site &s, bool skip_rskip_cols, FuseRule fuse) {
     ColProg cp;
     cp.col.resize(s.W.cols);
@@ -515,16 +505,12 @@ ColProg column_program(const Site &s, bool skip_rskip_cols, FuseRule fuse) {
                         }
                 }
             std::stable_sort(ents.begin(), ents.end(), [](const E &x, const E &y) { return x.key < y.key; });
-            size_t ngroups = 0, nouts = 0;
-            for (size_t i = 0; i < ents.size(); ++i) {
+            size_t ngroups = 0;
+            for (size_t i = 0; i < ents.size(); ++i)
                 if (i == 0 || ents[i].key != ents[i - 1].key) ++ngroups;
-                if (i == 0 || (ents[i].key >> 48) != (ents[i - 1].key >> 48)) ++nouts;
-            }
             bool fused = (fuse.mode == 2 && !ents.empty()) ||
                          (fuse.mode == 1 && ents.size() >= (size_t)fuse.min_entries &&
-                          (ents.size() >= (size_t)fuse.ratio * ngroups ||
-                           (ents.size() >= (size_t)2 * fuse.ratio * nouts &&
-                            2 * ents.size() >= (size_t)fuse.ratio * ngroups)));
+                          ents.size() >= (size_t)fuse.ratio * ngroups);
             if (!fused) {
                 for (int b1 : s.W.col_b1[b2])
                     for (auto &term : s.W.terms(b1, b2)) cp.col[b2].push_back({b1, term.op, term.scale, s.W.lspin[b1]});
