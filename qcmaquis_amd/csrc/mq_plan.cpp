@@ -720,60 +720,52 @@ TLay t_layout(const Site &s, const BLayout &L, PRP &prp, ColProg *cp, std::vecto
         const int al = s.lp_r[(size_t)lb * s.np + o.pout];
         return al >= 0 && s.x_of_r[al] >= 0 ? al : -1;
     };
-    // The sources of output o: each L block of each member row, the entries of one row
-    // summed; blocks whose every coupling vanishes are left out.
-    struct FSrc {
-        int at;   // [lb][in][lk]
-        int row;  // LA row of the block
-        double c;
-    };
-    auto list_sources = [&](const FOut &o, TaskVec<FSrc> &out) {
+    // f(place, LA row, coefficient) for every source of output o, place being [lb][in][lk]: each
+    // L block of each member row, the entries of one row summed; blocks whose every
+    // coupling vanishes are left out.
+    auto for_sources = [&](const FOut &o, auto &&f) {
         thread_local std::vector<double> tab;  // coupling [class][lk][lb], of SU(2)
         thread_local std::vector<char> have;
+        thread_local std::vector<int> out_r, in_r;  // right charges by lb, by lk
         const int ni = (int)o.in.size();
-        size_t most = 0;
-        for (auto &in : o.in)
-            for (size_t m = 0; m < in.mem.size(); ++m)
-                if (m == 0 || in.mem[m].b1 != in.mem[m - 1].b1) most += blk[in.mem[m].b1].size();
-        out.resize(most);
-        size_t n = 0;
+        out_r.resize(nl);
+        in_r.resize(nl);
+        for (int l = 0; l < nl; ++l) out_r[l] = right_out(o, l);
         for (int q = 0; q < ni; ++q) {
             const FIn &in = o.in[q];
+            for (int l = 0; l < nl; ++l) in_r[l] = right_in(in, l);
             if (s.su2) {
                 tab.resize(in.cls.size() * nl * nl);
                 have.assign(in.cls.size() * nl * nl, 0);
             }
             for (size_t m0 = 0; m0 < in.mem.size();) {
                 size_t m1 = m0;
-                while (m1 < in.mem.size() && in.mem[m1].b1 == in.mem[m0].b1) ++m1;
+                double w = 0.0;
+                for (; m1 < in.mem.size() && in.mem[m1].b1 == in.mem[m0].b1; ++m1) w += in.mem[m1].w;
                 for (auto &a : blk[in.mem[m0].b1]) {
-                    const int ar = right_in(in, a.lk), al = right_out(o, a.lb);
+                    const int ar = in_r[a.lk], al = out_r[a.lb];
                     if (ar < 0 || al < 0) continue;
-                    double c = 0.0;
-                    bool any = !s.su2;
-                    for (size_t m = m0; m < m1; ++m) {
-                        if (!s.su2) {
-                            c += in.mem[m].w;
-                            continue;
+                    double c = w;
+                    bool any = true;
+                    if (s.su2) {
+                        c = 0.0;
+                        any = false;
+                        for (size_t m = m0; m < m1; ++m) {
+                            const size_t at = ((size_t)in.mem[m].cls * nl + a.lk) * nl + a.lb;
+                            if (!have[at]) {
+                                tab[at] = factor(o, in.cls[in.mem[m].cls], a.lk, a.lb, ar, al);
+                                have[at] = 1;
+                            }
+                            any = any || tab[at] != 0.0;
+                            c += in.mem[m].w * tab[at];
                         }
-                        const size_t at = ((size_t)in.mem[m].cls * nl + a.lk) * nl + a.lb;
-                        if (!have[at]) {
-                            tab[at] = factor(o, in.cls[in.mem[m].cls], a.lk, a.lb, ar, al);
-                            have[at] = 1;
-                        }
-                        any = any || tab[at] != 0.0;
-                        c += in.mem[m].w * tab[at];
                     }
-                    if (any) out[n++] = {(a.lb * ni + q) * nl + a.lk, a.row, c};
+                    if (any) f((a.lb * ni + q) * nl + a.lk, a.row, c);
                 }
                 m0 = m1;
             }
         }
-        out.resize(n);
     };
-    // 1. (parallel) the sources of each output, its rows and their chunks.  The sources are
-    // kept for step 4: listing them is the larger part of both steps.
-    std::vector<TaskVec<FSrc>> srcs(ng);
     // a thread is worth starting (some 20 us) for about 4,096 sources; estimated from the
     // entries and the blocks per MPO row
     double work = 1.0;
@@ -783,15 +775,38 @@ TLay t_layout(const Site &s, const BLayout &L, PRP &prp, ColProg *cp, std::vecto
     for (auto &b : blk) nblk += b.size();
     work *= (double)nblk / std::max(nb1, 1);
     const int grain = (int)std::min(1e9, std::max(4.0, ng * 4096.0 / work));
+    // 1. (parallel) the sources of each output, its rows and their chunks.  Up to kKeepSrcs of
+    // them (256 MB) are kept for step 4, since listing them is the larger part of both steps in
+    // small plans (SU2U1 L=8 m=30: 1.4 ms each of 8.6); long lists (770 M at TwoU1 L=40 m=1024)
+    // are gone through twice, which costs less than their memory.
+    constexpr double kKeepSrcs = 16e6;
+    struct FSrc {
+        int at, row;
+        double c;
+    };
+    const bool keep = work <= kKeepSrcs;
+    std::vector<TaskVec<FSrc>> srcs(ng);
     parallel_for(
         ng,
         [&](int gi) {
             FOut &o = cp->fo[gi];
             thread_local std::vector<int> cnt;  // [lb][in][lk]
             const size_t ni = o.in.size();
-            list_sources(o, srcs[gi]);
             cnt.assign(ni * nl * nl, 0);
-            for (auto &x : srcs[gi]) ++cnt[x.at];
+            if (keep) {
+                size_t most = 0, n = 0;
+                for (auto &in : o.in)
+                    for (size_t m = 0; m < in.mem.size(); ++m)
+                        if (m == 0 || in.mem[m].b1 != in.mem[m - 1].b1) most += blk[in.mem[m].b1].size();
+                srcs[gi].resize(most);
+                for_sources(o, [&](int at, int row, double c) {
+                    srcs[gi][n++] = {at, row, c};
+                    ++cnt[at];
+                });
+                srcs[gi].resize(n);
+            } else {
+                for_sources(o, [&](int at, int, double) { ++cnt[at]; });
+            }
             for (int lb = 0; lb < nl; ++lb) {
                 const int al = right_out(o, lb);
                 if (al < 0) continue;
@@ -923,10 +938,14 @@ TLay t_layout(const Site &s, const BLayout &L, PRP &prp, ColProg *cp, std::vecto
                         k += s.lsize(c.lk);
                     }
                 }
-                for (auto &x : srcs[gi]) {
-                    const int lk = x.at % nl;
-                    comb->srcs[pos[x.at]++] = {t.la_off[lk] + x.row, t.Mtot[lk], x.c};
-                }
+                auto place_src = [&](int at, int row, double c) {
+                    const int lk = at % nl;
+                    comb->srcs[pos[at]++] = {t.la_off[lk] + row, t.Mtot[lk], c};
+                };
+                if (keep)
+                    for (auto &x : srcs[gi]) place_src(x.at, x.row, x.c);
+                else
+                    for_sources(o, place_src);
             },
             grain, 1);
     }
