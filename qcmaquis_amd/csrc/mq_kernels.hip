@@ -284,10 +284,11 @@ __device__ __forceinline__ void a_slot(int r, int &i, int &k) {
 // The plain operands' loads are unconditional, at addresses clamped into the operands:
 // rows and columns past the edge give results that are not stored, and k past the end is
 // zeroed before the stash (gemm_mask).  A load under a condition sits in a block of its
-// own; without them the T GEMM of the L=24 m=512 centre takes 745 against 786 us (BF16x3)
+// own; without them the T GEMM of the L=24 m=512 centre took 745 against 786 us (BF16x3)
 // and 768 against 797 (TwoU1, FP32), and FP64 the same 1,860.  The gathered form keeps
 // conditional loads (GATHER): there the columns past N and the empty row blocks are bytes
-// not read (FP64 1,291 against 1,392 us, BF16x3 561 against 611).
+// not read (FP64 1,291 against 1,392 us, BF16x3 561 against 611, before the B loads left
+// their addresses out of the registers; see gemm_fetch_b).
 template <int TM, int TN, class T, bool QUADS = false>
 __device__ __forceinline__ void gemm_fetch_a(const GemmGroup &g, const T *__restrict__ A, int m0, int k0, int kend,
                                              GemmStage<TM, TN, T> &st) {
@@ -754,9 +755,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(X3 ? 3
 // (T block or W-application strip) x RB.  Most C strips have a single source, one T block
 // times a coefficient (63 % of C at the L=24 m=512 centre, 85 % for TwoU1), and some
 // none; the W application wrote them to C and this GEMM read them back.  Gathering costs
-// the GEMM some time (source records, shorter runs: FP64 1,157 -> 1,291 us, BF16x3 500 ->
-// 561, TwoU1 FP32 640 -> 675) and takes the single-source strips out of the W
-// application (1,041 -> 338, 690 -> 198, 650 -> 27 us).
+// the GEMM some time (source records, shorter runs: FP64 1,157 -> 1,274 us, BF16x3 500 ->
+// 532, TwoU1 FP32 640 -> 652) and takes the single-source strips out of the W
+// application (1,041 -> 337, 690 -> 195, 650 -> 29 us).
 template <class T, bool X3>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 3 : 2)))
 k_gemm_gather(const GemmGroup *__restrict__ groups, const GemmTile *__restrict__ tiles, const T *__restrict__ A,
